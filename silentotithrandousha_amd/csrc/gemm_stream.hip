@@ -28,6 +28,9 @@
 // The epilogue's global stores are inline assembly (str_st*, stream.hpp): with stores pending
 // among the loads the compiler would wait for every load, and the ring would drain at each
 // round's end.
+//
+// COLS = 8 (four terms, launch_gemm_fine): chunks of up to 8 entries, MFMA column j = entry j % 8 of
+// term 2 m + j / 8, m = 0, 1; the two halves' sums are added once, in the epilogue.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -40,7 +43,7 @@ namespace moe {
 
 constexpr int kStrCompute = 4;                // compute wavefronts: one unit each per round
 constexpr int kStrWaves = kStrCompute + 1;    // and the B loader
-constexpr int kStrCols = 16;    // entries per chunk: one MFMA column group
+constexpr int kStrCols = 16;    // MFMA columns of a chunk (16 entries, or fewer with several terms each)
 constexpr int kStrMaxSeg = 32;  // chunks one workgroup's range may touch (the host checks)
 constexpr int kStrPos = 24;     // loop positions of a round (kGemmNs steps)
 static_assert(kGemmNs == kStrPos, "one loop position per record step");
@@ -49,10 +52,10 @@ constexpr int kStrBiasPos = 12; // position of a round whose loads include the u
 
 // The B loader's DMAs per position and its wait before each step (NSR real steps per round;
 // NSR = 24 takes any ns <= 24, steps from ns on loaded as in-range repeats and not computed).
-template <int NSR, int PB, int NT>
+template <int NSR, int PB, int NT, int COLS>
 struct StrLoader {
   using G = GemmRecT<NT>;
-  static constexpr int kPieces = (kStrCols * G::kStep + 1023) / 1024;  // 1 KB pieces of a chunk's B step
+  static constexpr int kPieces = (COLS * G::kStep + 1023) / 1024;  // 1 KB pieces of a chunk's B step
   static constexpr int kDma = 2 * kPieces;                             // two chunk areas per step
   static_assert(kStrPos % PB == 0 && PB >= 3, "ring slots fixed per position");
   // DMAs issued at position x: those of step x + PB - 1 (this round's or the next one's)
@@ -94,21 +97,24 @@ struct StrRound {
   int qf;               // the round's first chunk (segment index)
 };
 
-template <int MODE, int RT, int NSR, int PA, int PB, int NT>
+template <int MODE, int RT, int NSR, int PA, int PB, int NT, int COLS>
 __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_stream(GemmArgs a) {
   static_assert(MODE != GEMV_GATE_UP || RT == 4, "gate_up units are whole h blocks");
   static_assert(NSR == 23 || NSR == 24, "23 steps (K = 2880) or up to 24");
   static_assert(kStrPos % PA == 0 && PA >= 2, "A ring slots fixed per position");
-  using L = StrLoader<NSR, PB, NT>;
+  static_assert(COLS == 8 || COLS == kStrCols, "terms fill the columns that entries leave");
+  constexpr int TPM = kStrCols / COLS;  // terms per MFMA: column j = entry j % COLS, term j / COLS of a group of TPM
+  static_assert(NT % TPM == 0, "whole groups of terms");
+  using L = StrLoader<NSR, PB, NT, COLS>;
   using G = GemmRecT<NT>;
   constexpr int kPieces = L::kPieces, kBArea = kPieces * 1024;
   constexpr int QR = PA <= 4 ? 2 : 3;  // A-scale quads held at once
   static_assert((kStrPos / 4) % QR == 0, "a round's quads map to fixed scale slots");
   __shared__ __attribute__((aligned(1024))) uint8_t sB[PB][2][kBArea];
   __shared__ __attribute__((aligned(1024))) uint8_t sBd[1024];  // target of the absent second chunk's pieces
-  __shared__ __attribute__((aligned(16))) float s_stage[kStrCompute][MODE == GEMV_GATE_UP ? kStrCols * kStrRow : 4];
+  __shared__ __attribute__((aligned(16))) float s_stage[kStrCompute][MODE == GEMV_GATE_UP ? COLS * kStrRow : 4];
   __shared__ int s_seg[kStrMaxSeg][3];         // expert, first entry, entry count
-  __shared__ int s_row[kStrMaxSeg][kStrCols];  // B record row of each entry
+  __shared__ int s_row[kStrMaxSeg][COLS];  // B record row of each entry
   // local grouping: entry n's expert, then its grouped position; grouped entry -> token; the
   // experts' counts (then running ranks), first entries and the active list
   __shared__ int s_ge[MODE == GEMV_GATE_UP ? kLocalGroupMax : 1];
@@ -234,7 +240,7 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int r = 0; r < kR; r++) {
     if (64 * r + lane >= na) lo[r] = hi[r] = 0;
-    nc[r] = (hi[r] - lo[r] + kStrCols - 1) / kStrCols;
+    nc[r] = (hi[r] - lo[r] + COLS - 1) / COLS;
     int incl = nc[r];
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -265,8 +271,8 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
           const int hl = __builtin_ctzll(hit);
           const int e_ = __shfl(id[r], hl), l_ = __shfl(lo[r], hl), h_ = __shfl(hi[r], hl), s_ = __shfl(c0[r], hl);
           ex = e_;
-          beg = l_ + (ci - s_) * kStrCols;
-          cnt = min(kStrCols, h_ - beg);
+          beg = l_ + (ci - s_) * COLS;
+          cnt = min(COLS, h_ - beg);
         }
       }
       if (lane == 0) {
@@ -282,7 +288,7 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
     // issue their first weight loads, which need only the chunk table
     for (int q4 = 0; q4 < nseg; q4 += 4) {  // lane (q4 + lane / 16, entry j)
       const int q = q4 + g;
-      if (q < nseg) {
+      if (q < nseg && j < COLS) {
         const int beg = s_seg[q][1], cnt = s_seg[q][2];
         const int e = beg + min(j, max(cnt, 1) - 1);
         s_row[q][j] = local ? s_esrc[e] : (a.entry_src ? a.entry_src[e] : e);
@@ -332,7 +338,7 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int i = 0; i < L::kDma; i++) {
         const int ar = i / kPieces, pc = i % kPieces;
-        const int c = min(64 * pc + lane, kStrCols * G::kChunks - 1);
+        const int c = min(64 * pc + lane, COLS * G::kChunks - 1);
         real[i] = ar == 0 || t.two;
         const int qa = min(t.qf + ar, kStrMaxSeg - 1);
         off[i] = real[i] ? (uint32_t)s_row[qa][c / G::kChunks] * (uint32_t)G::kBytes + 16u * (c % G::kChunks) : 0u;
@@ -422,27 +428,38 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
       }
       if constexpr (p < NSR) {
         if (NSR == 23 || p < ns) {  // (NSR = 24: steps from ns on are repeats)
-          const uint8_t *eb = &sB[p % PB][0][0] + cur.area * kBArea + j * G::kStep;
-          i32x8 bv[NT];
+          const uint8_t *eb = &sB[p % PB][0][0] + cur.area * kBArea + (j % COLS) * G::kStep;
+          constexpr int NM = NT / TPM;  // MFMAs per weight chunk
+          const uint8_t *et = eb + (j / COLS) * G::kTermBytes;  // the lane's term of each group
+          i32x8 bv[NM];
 #pragma unroll
-          for (int tt = 0; tt < NT; tt++) {
-            const uint4 h = *reinterpret_cast<const uint4 *>(eb + tt * G::kTermBytes + 16 * g);
-            const uint2 tl = *reinterpret_cast<const uint2 *>(eb + tt * G::kTermBytes + 64 + 8 * g);
-            bv[tt] = i32x8{(int)h.x, (int)h.y, (int)h.z, (int)h.w, (int)tl.x, (int)tl.y, 0, 0};
+          for (int m = 0; m < NM; m++) {
+            const uint4 h = *reinterpret_cast<const uint4 *>(et + m * TPM * G::kTermBytes + 16 * g);
+            const uint2 tl = *reinterpret_cast<const uint2 *>(et + m * TPM * G::kTermBytes + 64 + 8 * g);
+            bv[m] = i32x8{(int)h.x, (int)h.y, (int)h.z, (int)h.w, (int)tl.x, (int)tl.y, 0, 0};
           }
-          const uint4 bsc = *reinterpret_cast<const uint4 *>(eb + NT * G::kTermBytes);
+          uint32_t bsc[NM];  // the E8M0 words of the lane's terms
+          if constexpr (TPM == 1) {
+            const uint4 w4 = *reinterpret_cast<const uint4 *>(eb + NT * G::kTermBytes);
+            const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+            for (int m = 0; m < NM; m++) bsc[m] = w[m];
+          } else {
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+              bsc[m] = *reinterpret_cast<const uint32_t *>(eb + NT * G::kTermBytes + 4 * (m * TPM + j / COLS));
+          }
           const StrSlot<RT> &sl = ring[p % PA];
           const uint32_t(&sa)[RT] = sw[(p / 4) % QR];
           const int sh = 8 * (p % 4);
 #pragma unroll
-          for (int tt = 0; tt < NT; tt++) {
-            const uint32_t wsc = tt == 0 ? bsc.x : (tt == 1 ? bsc.y : bsc.z);
-            const int sb = (int)(wsc >> (8 * g));
+          for (int m = 0; m < NM; m++) {
+            const int sb = (int)(bsc[m] >> (8 * g));
 #pragma unroll
             for (int r = 0; r < RT; r++) {
               const i32x8 A = {(int)sl.a[r].x, (int)sl.a[r].y, (int)sl.a[r].z, (int)sl.a[r].w, 0, 0, 0, 0};
               // cbsz 4: A is fp4 (E2M1); blgp 2: B is fp6 (E2M3)
-              acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, bv[tt], acc[r], 4, 2, 0, (int)(sa[r] >> sh), 0, sb);
+              acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, bv[m], acc[r], 4, 2, 0, (int)(sa[r] >> sh), 0, sb);
             }
           }
           // the step's MFMAs stay here (IR passes otherwise sink them towards the epilogue, keeping
@@ -463,6 +480,14 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
       }
       if constexpr (p == kStrPos - 1) {
         // ---- epilogue of this wavefront's unit of round k
+        if constexpr (TPM > 1) {  // the terms' columns of each entry
+#pragma unroll
+          for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              acc[r][i] = acc[r][i] + xor_lane<8>(acc[r][i]);
+            }
+        }
         if (cur.store) {
           if constexpr (MODE == GEMV_GATE_UP) {
             // lane (j, g) holds rows 16 r + 4 g .. + 3 of the group (gate = row 2i, up = row 2i + 1):
@@ -472,9 +497,12 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int r = 0; r < RT; r++) {
               const float4 b4 = bias[r];
-              *reinterpret_cast<float2 *>(st + j * kStrRow + 8 * r + 2 * g) =
-                  make_float2(swiglu_fast(acc[r][0] + b4.x, acc[r][1] + b4.y, a.limit),
-                              swiglu_fast(acc[r][2] + b4.z, acc[r][3] + b4.w, a.limit));
+              // (four terms: h is exact to 2^-18, so its last bits count)
+              const float2 h2 = NT > kGemmTerms ? make_float2(swiglu(acc[r][0] + b4.x, acc[r][1] + b4.y, a.limit),
+                                                              swiglu(acc[r][2] + b4.z, acc[r][3] + b4.w, a.limit))
+                                                : make_float2(swiglu_fast(acc[r][0] + b4.x, acc[r][1] + b4.y, a.limit),
+                                                              swiglu_fast(acc[r][2] + b4.z, acc[r][3] + b4.w, a.limit));
+              if (COLS == kStrCols || j < COLS) *reinterpret_cast<float2 *>(st + j * kStrRow + 8 * r + 2 * g) = h2;
             }
             if (lane < cur.cnt) {
               float v[32];
@@ -537,11 +565,11 @@ bool gemm_stream_local_ok(const GemmArgs &a);
 // Whether the launch fits the streamed kernel: whole units, K <= 3072, at least 3 units per chunk
 // (4 consecutive units then touch at most two chunks) and, from the host's upper bound on the
 // chunks (entries / 16 + active experts), at most kStrMaxSeg chunks per workgroup range.
-static bool gemm_stream_fits(const GemmArgs &a, int rt, int n_wg) {
+static bool gemm_stream_fits(const GemmArgs &a, int rt, int n_wg, int cols = kStrCols) {
   if (a.d.tiles % rt || a.d.ns > (uint32_t)kGemmNs || a.max_active > kMaxExperts || n_wg % 8) return false;
   const long long gu = a.d.tiles / rt;
   if (gu < 3) return false;
-  const long long nc = (long long)(a.n_entries / kStrCols) + std::min<long long>(a.max_active, (long long)a.n_entries);
+  const long long nc = (long long)(a.n_entries / cols) + std::min<long long>(a.max_active, (long long)a.n_entries);
   if (gu * nc > INT32_MAX / 2) return false;
   const long long per = (gu * nc + n_wg - 1) / n_wg;
   const long long segs = per > 0 ? (per + gu - 2) / gu + 1 : 1;
@@ -551,6 +579,21 @@ static bool gemm_stream_fits(const GemmArgs &a, int rt, int n_wg) {
 static int stream_cus();
 bool gemm_stream_local_ok(const GemmArgs &a) {
   return a.n_entries <= (size_t)kLocalGroupMax && a.terms == kGemmTerms && gemm_stream_fits(a, 4, stream_cus());
+}
+
+// Entries per chunk of the four-term form: two of the four terms of eight entries fill the 16 MFMA
+// columns, so a weight chunk feeds two MFMAs and the loader moves half the records of a 16-entry
+// chunk. Measured (20B / 120B layer, us): 7 tokens 68.7 against 73.5 with 16 entries and 68.0 with
+// 4; 31 tokens 96.1 against 104.3 and 113.4 (experts of more than 4 entries stream twice); 120B at
+// 127 tokens 336 against 356 and 421.
+constexpr int kFineCols = 8;
+
+bool gemm_fine_fits(const GemmArgs &gu, const PackDims &dn) {
+  GemmArgs d = gu;
+  d.d = dn;
+  const int n_wg = stream_cus();
+  return gu.n_entries > 0 && gu.n_entries <= (size_t)kLocalGroupMax && gemm_stream_fits(gu, 4, n_wg, kFineCols) &&
+         gemm_stream_fits(d, 2, n_wg, kFineCols);
 }
 
 static int stream_cus() {
@@ -567,12 +610,12 @@ static int stream_cus() {
   return c;
 }
 
-template <int MODE, int RT, int PA, int PB, int NT>
+template <int MODE, int RT, int PA, int PB, int NT, int COLS = kStrCols>
 static hipError_t launch_stream_rt(const GemmArgs &a, hipStream_t s, int n_wg) {
   if (a.d.ns == 23)
-    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 23, PA, PB, NT>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 23, PA, PB, NT, COLS>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
   else
-    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 24, PA, PB, NT>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 24, PA, PB, NT, COLS>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
   return hipGetLastError();
 }
 
@@ -594,6 +637,20 @@ hipError_t launch_gemm_stream(GemvMode mode, const GemmArgs &a, hipStream_t s, b
   if (alt)
     return one ? launch_stream_rt<GEMV_DOWN, 2, 6, 6, 1>(a, s, n_wg) : launch_stream_rt<GEMV_DOWN, 2, 6, 6, kGemmTerms>(a, s, n_wg);
   return one ? launch_stream_rt<GEMV_DOWN, 2, 8, 4, 1>(a, s, n_wg) : launch_stream_rt<GEMV_DOWN, 2, 8, 4, kGemmTerms>(a, s, n_wg);
+}
+
+// The four-term form (experts averaging fewer than 4 entries). The weight stream bounds it: at 120B
+// x 48 tokens gate_up reads 0.88 GB in 151 us (5.9 TB/s). A register rings of 4 (gate_up) and 8
+// (down) steps, as the three-term form's 3 and 8. Against the per-tile GEMV on bf16 hi + lo
+// operands, whose weight decode bounds it (us per layer): 20B at 2 tokens 49.8 -> 40.8, 8 tokens
+// 123.7 -> 70.4, 31 tokens 193.4 -> 96.1; 120B at 16 tokens 226.5 -> 144.0, 48 tokens 489 -> 251,
+// 127 tokens 638 -> 336.
+hipError_t launch_gemm_fine(GemvMode mode, const GemmArgs &a, hipStream_t s) {
+  const int n_wg = stream_cus();
+  if (!a.n_entries) return hipSuccess;
+  if (a.terms != kFineTerms || !gemm_stream_fits(a, mode == GEMV_GATE_UP ? 4 : 2, n_wg, kFineCols)) return hipErrorInvalidValue;
+  return mode == GEMV_GATE_UP ? launch_stream_rt<GEMV_GATE_UP, 4, 4, 4, kFineTerms, kFineCols>(a, s, n_wg)
+                              : launch_stream_rt<GEMV_DOWN, 2, 8, 4, kFineTerms, kFineCols>(a, s, n_wg);
 }
 
 }  // namespace moe

@@ -107,7 +107,8 @@ __host__ __device__ constexpr int route_hp(int H) { return ((H + 63) / 64 + 7) /
 // E <= 128: block_topk's arithmetic), or for larger k the block runs block_topk per token.
 // With xrec the block also writes its tokens' grouped-GEMM records; with bucket_ticket the last
 // block to finish groups every entry by expert (bucket_block) in its free x staging area.
-template <int KI, int TB>
+// NT: the records' terms.
+template <int KI, int TB, int NT>
 __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   __shared__ float s_logit[TB][kMaxExperts];
   __shared__ float s_p[kMaxExperts];
@@ -184,10 +185,7 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
         xv[4 * q + 2] = k0 + 4 * q + 2 < H ? x4.z : 0.0f;
         xv[4 * q + 3] = k0 + 4 * q + 3 < H ? x4.w : 0.0f;
       }
-      if (a.rec_terms == 1)
-        rec_split_block<1>(xv, blk, a.xrec + (size_t)(t0 + tb) * GemmRecT<1>::kBytes);
-      else
-        rec_split_block<kGemmTerms>(xv, blk, a.xrec + (size_t)(t0 + tb) * GemmRec::kBytes);
+      rec_split_block<NT>(xv, blk, a.xrec + (size_t)(t0 + tb) * GemmRecT<NT>::kBytes);
     }
   };
   if constexpr (KI > 0) {
@@ -417,21 +415,29 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   }
 }
 
+template <int KI, int TB, int NT>
+static hipError_t launch_route_tb(const RouteArgs &a, size_t hp, hipStream_t s) {
+  if (TB * hp > 65536) {  // more than the default 64 KB of dynamic LDS
+    static DynLdsOnce once;
+    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, TB, NT>), TB * hp);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_route<KI, TB, NT>), dim3((unsigned)((a.T + TB - 1) / TB)), dim3(kRouteThreads), TB * hp, s, a);
+  return hipGetLastError();
+}
+
 template <int KI>
 static hipError_t launch_route_ki(const RouteArgs &a, int nq, hipStream_t s) {
   const size_t hp = (size_t)nq * 8 * 64 * sizeof(float);
+  const int nt = a.xrec ? a.rec_terms : kGemmTerms;
   if (a.T >= 2048 && kRouteTokens * hp <= 144 * 1024) {
-    // TB tokens of x may exceed the default 64 KB of dynamic LDS
-    static DynLdsOnce once;
-    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, kRouteTokens>),
-                                        kRouteTokens * hp);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_route<KI, kRouteTokens>), dim3((unsigned)((a.T + kRouteTokens - 1) / kRouteTokens)),
-                       dim3(kRouteThreads), kRouteTokens * hp, s, a);
-  } else {
-    hipLaunchKernelGGL((k_route<KI, 1>), dim3((unsigned)a.T), dim3(kRouteThreads), hp, s, a);
+    if (nt == 1) return launch_route_tb<KI, kRouteTokens, 1>(a, hp, s);
+    if (nt == kGemmTerms) return launch_route_tb<KI, kRouteTokens, kGemmTerms>(a, hp, s);
   }
-  return hipGetLastError();
+  if (nt == 1) return launch_route_tb<KI, 1, 1>(a, hp, s);
+  if (nt == kFineTerms) return launch_route_tb<KI, 1, kFineTerms>(a, hp, s);
+  if (nt == kGemmTerms) return launch_route_tb<KI, 1, kGemmTerms>(a, hp, s);
+  return hipErrorInvalidValue;
 }
 
 bool route_bucket_fits(int H, int E) { return 18 * E <= route_hp(H); }

@@ -48,7 +48,7 @@ struct RouteArgs {
   float *wts;            // [T, k]
   uint16_t *xsplit;      // [T, 2, H] bf16 hi / lo
   uint8_t *xrec;         // [T] GemmRecT<rec_terms> records of x (grouped GEMM operands; H <= 128 kGemmNs)
-  int rec_terms;         // kGemmTerms (exact split) or 1 (one MXFP6 term per value)
+  int rec_terms;         // kGemmTerms or kFineTerms (exact splits) or 1 (one MXFP6 term per value)
   int fuse_bucket;       // T == 1: also write the expert list
   int32_t *n_active, *active_ids, *active_off, *entry_src, *pos;
   uint32_t *bucket_ticket;  // T > 1: zeroed counter; the last block buckets (route_bucket_fits)
@@ -83,10 +83,12 @@ constexpr int kTerms = 4;
 // i = E8M0 of block 4s+i] (4 NT bytes) and pad bytes to 16. A step is kChunks 16-byte chunks:
 // chunk 6t + b = the first 16 bytes of block b, chunk 6t + 4 + (b >> 1) = the last 8 bytes of
 // blocks b and b ^ 1, chunk 6 NT = the scales (the grouped GEMM stages them chunk by chunk).
-// Blocks past the row are zero. NT = kGemmTerms: the exact split (the default); NT = 1: the
-// quantized-activation mode (one MXFP6 term per value).
+// Blocks past the row are zero. NT = kGemmTerms: the exact split (the default); NT = kFineTerms: one
+// term more (2^-18 of a block's maximum), for batches whose experts average fewer than 4 entries;
+// NT = 1: the quantized-activation mode (one MXFP6 term per value).
 constexpr int kGemmNs = 24;
 constexpr int kGemmTerms = 3;
+constexpr int kFineTerms = 4;
 template <int NT>
 struct GemmRecT {
   static constexpr int kNT = NT;
@@ -99,7 +101,7 @@ struct GemmRecT {
     return s * kStep + t * kTermBytes + (d < 4 ? 16 * b + 4 * d : 64 + 8 * b + 4 * (d - 4));
   }
   MOE_HD static constexpr int scale(int s, int t) { return s * kStep + NT * kTermBytes + 4 * t; }
-  static_assert(NT >= 1 && NT <= 3 && kStep % 16 == 0 && kChunks == 6 * NT + 1, "record chunks");
+  static_assert(NT >= 1 && NT <= 4 && kStep % 16 == 0 && kChunks == 6 * NT + 1, "record chunks");
 };
 using GemmRec = GemmRecT<kGemmTerms>;
 
@@ -119,7 +121,7 @@ struct GemmArgs {
   int n_row_blocks;          // set by launch_gemm_fp8: row blocks of the launch
   int n_tiles;               //                         row blocks x column tiles
   int n_blocks;              //                         workgroups of the tile order (>= n_tiles)
-  int terms;                 // E2M3 terms per activation value: kGemmTerms, or 1 (quantized mode)
+  int terms;                 // E2M3 terms per activation value: kGemmTerms, 1 (quantized mode) or kFineTerms
   int32_t *queue;            // tile queue of the persistent pipelined step: 10 counters, zero between launches
   // Local grouping (the streamed gate_up GEMM of a batch of at most kLocalGroupMax entries): with
   // group_idx set (the top-k indices [T][group_k] over group_E experts, -1 for a dropped slot)
@@ -138,6 +140,11 @@ hipError_t launch_gemm_fp8(GemvMode mode, const GemmArgs &a, hipStream_t s);
 // The streamed form for batches of a few entries per expert (gemm_stream.hip); hipErrorNotSupported
 // when the launch does not fit it.
 hipError_t launch_gemm_stream(GemvMode mode, const GemmArgs &a, hipStream_t s, bool alt);
+// The streamed form with kFineTerms terms, for batches whose experts average fewer than 4 entries
+// (activations to 2^-18 of a block's maximum); gemm_fine_fits: whether both GEMMs of the layer
+// (gu: the gate_up arguments; dn: the down matrix) and its local grouping take this batch.
+bool gemm_fine_fits(const GemmArgs &gu, const PackDims &dn);
+hipError_t launch_gemm_fine(GemvMode mode, const GemmArgs &a, hipStream_t s);
 // The wide streamed form for batches of tens of entries per expert (gemm_wide.hip): every weight
 // tile streams once per group of up to 5 16-entry chunks; hipErrorNotSupported when the launch
 // does not fit it.

@@ -87,7 +87,13 @@ struct Work {
   int32_t *idx, *n_active, *active_ids, *active_off, *entry_src, *pos;
   int32_t *blk_count, *rank;  // the router's grouping: per-block expert counts, per-entry ranks
   size_t hrec_bytes;     // bytes of hrec, which must hold zeros where no kernel writes
+  uint8_t *xfine, *hfine;  // the same with kFineTerms terms (small batches)
+  size_t hfine_bytes;
 };
+
+// Which activation operands a workspace holds: every path's (a context's own workspace), or those
+// of one path (the scratch array of the allocation-free forward).
+enum WorkFor { WORK_ALL, WORK_FINE, WORK_COARSE };
 
 enum {
   K_ROUTE = 0, K_BUCKET, K_GATE_UP, K_DOWN, K_COMBINE, K_DECODE_GATE_UP, K_DECODE_DOWN,
@@ -209,8 +215,13 @@ size_t router_bytes(size_t H, size_t E) { return E * 64 * router_kip(H) * 2; }
 // Lays out the per-call workspace of T tokens, top-k k and E experts at `b` (nullptr: sizes
 // only) and returns its bytes. host_io adds the staging rows of host-pointer calls (x, y) and
 // the normalised rows of the unfused block forward (xn).
-size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size_t I, bool host_io) {
+// what: with WORK_FINE only the operands of the four-term small-batch GEMM, with WORK_COARSE those
+// of the other paths.
+size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size_t I, bool host_io, WorkFor what) {
   const size_t N = T * k;
+  // the four-term GEMM takes batches of fewer than 4 E entries
+  const size_t NF = what == WORK_COARSE ? 0 : std::min(N, 4 * E), TF = what == WORK_COARSE ? 0 : std::min(T, 4 * E);
+  const size_t NC = what == WORK_FINE ? 0 : N, TC = what == WORK_FINE ? 0 : T;
   size_t off = 0;
   auto take = [&](size_t bytes) -> char * {
     const size_t o = off;
@@ -223,8 +234,8 @@ size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size
   w.logits = (float *)take(T * E * 4);
   w.wts = (float *)take(N * 4);
   w.o = (float *)take(N * H * 4);
-  w.xsplit = (uint16_t *)take(T * 2 * H * 2);
-  w.hsplit = (uint16_t *)take(N * 2 * I * 2);
+  w.xsplit = (uint16_t *)take(TC * 2 * H * 2);
+  w.hsplit = (uint16_t *)take(NC * 2 * I * 2);
   w.idx = (int32_t *)take(N * 4);
   w.n_active = (int32_t *)take(4);
   w.active_ids = (int32_t *)take(E * 4);
@@ -233,9 +244,13 @@ size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size
   w.pos = (int32_t *)take(N * 4);
   w.blk_count = (int32_t *)take(T * E * 4);  // router blocks <= T
   w.rank = (int32_t *)take(N * 4);
-  w.xrec = (uint8_t *)take(T * GemmRec::kBytes);
-  w.hrec_bytes = N * GemmRec::kBytes;
+  w.xrec = (uint8_t *)take(TC * GemmRec::kBytes);
+  w.xfine = (uint8_t *)take(TF * GemmRecT<kFineTerms>::kBytes);
+  // the h records last, one after the other: cleared together
+  w.hrec_bytes = NC * GemmRec::kBytes;
   w.hrec = (uint8_t *)take(w.hrec_bytes);
+  w.hfine_bytes = NF * GemmRecT<kFineTerms>::kBytes;
+  w.hfine = (uint8_t *)take(w.hfine_bytes);
   return off;
 }
 
@@ -251,10 +266,10 @@ int ensure_work(moe_ctx *c, size_t T, size_t k, size_t E) {
   // workspace (the next call sizes it again) and never pointers into freed memory
   c->w = Work{};
   c->work_T = c->work_k = c->work_E = 0;
-  RETURN_IF(c->work.ensure(carve_work(w, nullptr, T, k, E, c->H, c->I, true)));
-  carve_work(w, (char *)c->work.p, T, k, E, c->H, c->I, true);
+  RETURN_IF(c->work.ensure(carve_work(w, nullptr, T, k, E, c->H, c->I, true, WORK_ALL)));
+  carve_work(w, (char *)c->work.p, T, k, E, c->H, c->I, true, WORK_ALL);
   // h records are written block by block; their padding past I must read as zeros
-  HIP_TRY(hipMemset(w.hrec, 0, w.hrec_bytes));
+  HIP_TRY(hipMemset(w.hrec, 0, al(w.hrec_bytes) + w.hfine_bytes));
   c->w = w;
   c->work_T = T;
   c->work_k = k;
@@ -409,6 +424,27 @@ int set_single_token_list(moe_ctx *c, size_t n, const int32_t *ids) {
   return MOE_OK;
 }
 
+// The gate_up arguments that the grouped GEMM of a layer's batch starts from.
+GemmArgs gemm_args(const moe_ctx *c, const Layer &Ly, size_t T, size_t k) {
+  GemmArgs ga{};
+  ga.base = (const uint8_t *)Ly.experts.p;
+  ga.stride = c->L.stride;
+  ga.limit = c->clamp;
+  ga.max_active = (int)std::min(Ly.n_experts, T * k);
+  ga.n_entries = T * k;
+  ga.d = c->L.gu;
+  return ga;
+}
+
+// Whether a batch runs the four-term streamed GEMM: experts averaging fewer than 4 entries, where
+// the weights are read about once per entry and the three-term split of the larger batches would
+// be less exact than the bf16 hi + lo operands of the GEMV path that it replaces.
+bool takes_fine(const moe_ctx *c, const Layer &Ly, size_t T, size_t k, const float *x) {
+  return c->batch_gemm == 1 && T > 1 && T * k < 4 * Ly.n_experts && c->L.gu.ns <= (uint32_t)kGemmNs &&
+         c->L.dn.ns <= (uint32_t)kGemmNs && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+         gemm_fine_fits(gemm_args(c, Ly, T, k), c->L.dn);
+}
+
 // norm: the block forward (RMSNorm of x before, x + result after); the one-launch decode fuses
 // both, the other paths run k_rmsnorm into the workspace first and k_add_rows last.
 // w: the workspace, sized for (T, k, E) by the caller (ensure_work, or the scratch array of the
@@ -514,12 +550,13 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   // the grouped GEMM (16- to 64-entry column tiles) pays off once experts average a few
   // entries; smaller batches stream each weight tile through the GEMV kernels, which read the
   // bf16 hi + lo split of x that the router writes
-  const bool use_gemm = c->batch_gemm && T > 1 && (c->batch_gemm == 2 || T * k >= 4 * E) &&
-                        c->L.gu.ns <= (uint32_t)kGemmNs && c->L.dn.ns <= (uint32_t)kGemmNs &&
-                        (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const bool fine = w.hfine && takes_fine(c, Ly, T, k, x);
+  const bool use_gemm = fine || (c->batch_gemm && T > 1 && (c->batch_gemm == 2 || T * k >= 4 * E) &&
+                                 c->L.gu.ns <= (uint32_t)kGemmNs && c->L.dn.ns <= (uint32_t)kGemmNs &&
+                                 (reinterpret_cast<uintptr_t>(x) & 15) == 0);
   ra.xsplit = use_gemm ? nullptr : w.xsplit;
-  ra.xrec = use_gemm ? w.xrec : nullptr;  // the router writes the GEMM's activation records
-  ra.rec_terms = c->act_quant ? 1 : kGemmTerms;
+  ra.xrec = fine ? w.xfine : use_gemm ? w.xrec : nullptr;  // the router writes the GEMM's activation records
+  ra.rec_terms = fine ? kFineTerms : c->act_quant ? 1 : kGemmTerms;
   ra.fuse_bucket = T == 1;
   ra.n_active = w.n_active;
   ra.active_ids = w.active_ids;
@@ -529,32 +566,27 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   const int max_active = (int)std::min(E, T * k);
   GemmArgs ga{}, gu{};
   if (use_gemm) {
-    const size_t N = T * k;
-    ga.base = (const uint8_t *)Ly.experts.p;
-    ga.stride = c->L.stride;
+    ga = gemm_args(c, Ly, T, k);
     ga.n_active = w.n_active;
     ga.active_ids = w.active_ids;
     ga.active_off = w.active_off;
-    ga.limit = c->clamp;
-    ga.max_active = max_active;
-    ga.n_entries = N;
     ga.shape = c->gemm_shape;
     ga.band = c->gemm_band;  // default: gate_up in workgroup order, down in XCD bands of 1 row block
-    ga.terms = c->act_quant ? 1 : kGemmTerms;
+    ga.terms = ra.rec_terms;
     ga.queue = (int32_t *)c->gemm_queue.p;
     gu = ga;
     gu.mat_off = c->L.gu_off;
     gu.bias_off = c->L.gub_off;
     gu.d = c->L.gu;
     gu.entry_src = w.entry_src;
-    gu.brec = w.xrec;
-    gu.out = w.hrec;
+    gu.brec = ra.xrec;
+    gu.out = fine ? w.hfine : w.hrec;
   }
   // small batches on the streamed gate_up GEMM: its workgroups group the entries by expert
   // themselves (one round trip for the top-k indices, where the router's grouping took a
   // grid-wide ticket and a pass of its last block, and the GEMM two dependent round trips for
   // the lists and entry_src); its workgroup 0 writes the lists for the down GEMM and the combine
-  const bool local_group = use_gemm && c->local_group && gemm_gate_up_groups_locally(gu);
+  const bool local_group = use_gemm && c->local_group && (fine || gemm_gate_up_groups_locally(gu));
   if (local_group) {
     gu.group_idx = w.idx;
     gu.group_k = (int)k;
@@ -576,7 +608,8 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
                            w.active_off, w.entry_src, w.pos, s);
     }));
   if (use_gemm) {
-    RETURN_IF(timed(c, K_GATE_UP, s, [&] { return launch_gemm_fp8(GEMV_GATE_UP, gu, s); }));
+    auto gemm = fine ? launch_gemm_fine : launch_gemm_fp8;
+    RETURN_IF(timed(c, K_GATE_UP, s, [&] { return gemm(GEMV_GATE_UP, gu, s); }));
     GemmArgs dn = ga;
     if (!c->gemm_band) dn.band = 1;
     if (c->gemm_shape_down) dn.shape = c->gemm_shape_down;
@@ -584,9 +617,9 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
     dn.bias_off = c->L.dnb_off;
     dn.d = c->L.dn;
     dn.entry_src = nullptr;
-    dn.brec = w.hrec;
+    dn.brec = (const uint8_t *)gu.out;
     dn.out = w.o;
-    RETURN_IF(timed(c, K_DOWN, s, [&] { return launch_gemm_fp8(GEMV_DOWN, dn, s); }));
+    RETURN_IF(timed(c, K_DOWN, s, [&] { return gemm(GEMV_DOWN, dn, s); }));
   } else {
     RETURN_IF(run_experts(c, w, (const uint8_t *)Ly.experts.p, max_active, (int)std::min(T, (size_t)1 << 30), s));
   }
@@ -1022,16 +1055,22 @@ int moe_layer_forward_device_noalloc(moe_ctx *c, size_t layer, const float *x, s
   if (!c->scratch) return fail(MOE_ERR_STATE, "no scratch array address for device %d", c->dev);
   const size_t E = c->layers[layer].n_experts;
   Work w{};
-  const size_t need = carve_work(w, nullptr, T, k, E, c->H, c->I, false);
+  // a batch of the four-term GEMM whose operands the array does not hold takes the other path
+  WorkFor what = takes_fine(c, c->layers[layer], T, k, x) ? WORK_FINE : WORK_COARSE;
+  if (what == WORK_FINE && carve_work(w, nullptr, T, k, E, c->H, c->I, false, what) > noalloc_scratch_bytes()) what = WORK_COARSE;
+  const size_t need = carve_work(w, nullptr, T, k, E, c->H, c->I, false, what);
   if (need > noalloc_scratch_bytes())
     return fail(MOE_ERR_INVALID,
                 "%zu tokens at top-%zu over %zu experts need %zu bytes of workspace; the allocation-free "
                 "forward's scratch holds %zu (use moe_layer_forward_device)",
                 T, k, E, need, noalloc_scratch_bytes());
-  carve_work(w, (char *)c->scratch, T, k, E, c->H, c->I, false);
+  carve_work(w, (char *)c->scratch, T, k, E, c->H, c->I, false, what);
   const hipStream_t s = pick(c, stream);
   // the array keeps the previous call's contents: the h records' padding must read as zeros
-  HIP_TRY(launch_zero(w.hrec, w.hrec_bytes, s));
+  if (what == WORK_FINE)
+    HIP_TRY(launch_zero(w.hfine, w.hfine_bytes, s));
+  else
+    HIP_TRY(launch_zero(w.hrec, w.hrec_bytes, s));
   return forward_device(c, w, layer, x, T, k, y, s);
 }
 

@@ -1,0 +1,133 @@
+"""The four-term streamed GEMM that batches of fewer than 4 entries per expert take by default:
+against the fp32 oracle and against the per-tile GEMV path (bf16 hi + lo operands) it stands in
+for, at the edges of its 8-entry chunks and over ragged shapes."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from silentotithrandousha_amd import DeviceBuffer, GpuMoeDispatcher
+from silentotithrandousha_amd import synthetic as syn
+from silentotithrandousha_amd._ffi import check, lib
+from tests.helpers import assert_rel_l2, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# The GEMV's operands are within 2^-17 of each value, the four terms within 2^-18 of each block's
+# maximum: their products differ by about 1e-5 relative on these layers, whose pre-activations the
+# SwiGLU passes on without the large gains of wider scales.
+GEMV_TOL = 4e-5
+
+
+def _pair(d, x, k):
+    got = d.layer_forward(0, x, k)
+    d.set_batch_gemm(0)
+    ref = d.layer_forward(0, x, k)
+    d.set_batch_gemm(1)
+    return got, ref
+
+
+# H, I, E, k, T, router sigma: one and two K-step quads, K not a multiple of 128, the smallest shape the
+# streamed form takes (3 units per chunk) and one it refuses (64), 23 and 24 steps, 256 experts,
+# top-1, experts of 1 to 8, 9 and 17 entries (a large router spread sends every token to the
+# same experts), the largest average below 4
+CASES = [(96, 96, 8, 2, 5, 0.1), (64, 64, 8, 4, 3, 0.1), (160, 224, 8, 1, 31, 0.1), (512, 512, 64, 4, 50, 0.1),
+         (2880, 2880, 8, 4, 2, 0.1), (3072, 1056, 8, 4, 7, 0.1), (256, 3072, 32, 4, 31, 0.1),
+         (256, 128, 256, 4, 255, 0.1), (256, 256, 32, 4, 8, 40.0), (256, 256, 32, 4, 9, 40.0),
+         (256, 256, 32, 4, 17, 40.0)]
+
+
+@pytest.mark.parametrize("H,I,E,k,T,sigma", CASES)
+def test_small_batch_matches_oracle_and_gemv(orc, H, I, E, k, T, sigma):
+    assert T * k < 4 * E
+    L = syn.make_layer(H, I, E, seed=600 + T + H, scale_lo=117, scale_hi=121, router_sigma=sigma)
+    d = GpuMoeDispatcher(H, I, 7.0)
+    try:
+        d.preload_layer(0, L)
+        x = syn.hidden(T, H, seed=601 + T)
+        if sigma > 1:
+            x = x[:1] + 1e-3 * x  # tokens alike: the same experts for all of them
+        got, ref = _pair(d, x, k)
+        want, _, idx, _ = orc.moe_layer(x, L, k)
+        gidx, _ = d.router_topk(0, x, k)
+        assert np.array_equal(gidx, idx)
+        if sigma > 1:
+            assert np.bincount(idx[idx >= 0].ravel()).max() == T
+        e_new, e_gemv = assert_rel_l2(got, want, "four terms", 2e-5), assert_rel_l2(ref, want, "GEMV", 2e-5)
+        print(f"oracle: four terms {e_new:.2e}, GEMV {e_gemv:.2e}; apart {rel_l2(got, ref):.2e}")
+        assert rel_l2(got, ref) < GEMV_TOL
+        d.set_local_group(0)  # grouped by the router instead of the GEMM's workgroups
+        assert np.array_equal(d.layer_forward(0, x, k), got)
+    finally:
+        d.close()
+
+
+def test_small_batch_outliers_and_extremes(orc):
+    """Activations that a block scale serves worst: one value of a block a thousand times the rest,
+    magnitudes from 2^-100 to 2^60, zero rows, and a non-finite value (NaN in its token alone)."""
+    H, I, E, k = 512, 256, 16, 2
+    L = syn.make_layer(H, I, E, seed=640, scale_lo=117, scale_hi=121, router_sigma=0.1)
+    x = syn.hidden(9, H, seed=641)
+    x[0, ::32] *= 1000.0
+    x[1] *= np.float32(2.0**-100)
+    x[2, :64] *= np.float32(2.0**60)
+    x[3] = 0.0
+    d = GpuMoeDispatcher(H, I, 7.0)
+    try:
+        d.preload_layer(0, L)
+        got, ref = _pair(d, x, k)
+        want = orc.moe_layer(x, L, k)[0]
+        for t in range(9):
+            assert_rel_l2(got[t], want[t], f"token {t}", 1e-4)
+            assert rel_l2(got[t], ref[t]) < 1e-4
+        x[4, 7] = np.nan
+        bad = d.layer_forward(0, x, k)
+        assert not np.isfinite(bad[4]).any()
+        keep = [t for t in range(9) if t != 4]
+        assert np.array_equal(bad[keep], got[keep])
+    finally:
+        d.close()
+
+
+def test_small_batch_adaptive_unaligned_and_replayed(orc):
+    """Adaptive top-k's dropped slots; an x that is not 16-byte aligned (the GEMV path); a graph
+    captured after one eager call, replayed between eager calls of other sizes."""
+    H, I, E = 256, 128, 32
+    L = syn.make_layer(H, I, E, seed=650, scale_lo=117, scale_hi=121, router_sigma=0.2)
+    d = GpuMoeDispatcher(H, I, 7.0)
+    try:
+        d.preload_layer(0, L)
+        x = syn.hidden(20, H, seed=651)
+        d.set_adaptive_topk(True, 1, 0.7, 0.4, 0.85)
+        want, _, idx, _ = orc.moe_layer(x, L, 4, adaptive=orc.Adaptive(1, 1, 0.7, 0.4, 0.85))
+        assert (idx < 0).any()
+        got, ref = _pair(d, x, 4)
+        assert_rel_l2(got, want, "adaptive", 2e-5)
+        assert rel_l2(got, ref) < GEMV_TOL
+        d.set_adaptive_topk(False)
+        d.layer_forward(0, syn.hidden(123, H, seed=652), 4)  # the largest call first: the graph's workspace stays
+        eager = d.layer_forward(0, x, 4)
+        flat = DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+        y = DeviceBuffer(x.nbytes)
+        check(lib().moe_layer_forward_device(d.ctx, 0, ctypes.c_void_p(flat.ptr + 4), 20, 4, ctypes.c_void_p(y.ptr), None))
+        d.synchronize()
+        d.set_batch_gemm(0)
+        assert np.array_equal(y.download(np.float32, x.shape), d.layer_forward(0, x, 4))
+        d.set_batch_gemm(1)
+        xd, g = DeviceBuffer.from_array(x), ctypes.c_void_p()
+        check(lib().moe_graph_begin(d.ctx))
+        try:
+            d.layer_forward_device(0, xd, 20, 4, y)
+        finally:
+            check(lib().moe_graph_end(d.ctx, ctypes.byref(g)))
+        try:
+            for rep in range(3):
+                check(lib().moe_memset_device(ctypes.c_void_p(y.ptr), 0xFF, x.nbytes))
+                check(lib().moe_graph_launch(d.ctx, g))
+                d.synchronize()
+                assert np.array_equal(y.download(np.float32, x.shape), eager), f"replay {rep}"
+                d.layer_forward(0, syn.hidden(3 + 60 * rep, H, seed=660 + rep), 4)
+        finally:
+            check(lib().moe_graph_destroy(g))
+    finally:
+        d.close()
