@@ -1,10 +1,12 @@
 // Beaver-triple generation over p = 2^31 - 1 for gfx950 (include/beaver32.h): the GPU backend
 // GpuTripleGen32 of the reference (src/gpu/mod.rs:511-1012; kernels shader32.metal:75-167).
 //
-// A thread produces triple j of 16 rounds 64 apart, so each pass of a wavefront stores 64
-// consecutive words of each output array; a block takes 1024 whole rounds. The field products
-// are exact 32 x 32 -> 64-bit multiplies folded by 2^31 = 1 (mod p), those by the parties'
-// evaluation points 1..8 sums of 31-bit rotations; every value is kept in [0, p).
+// One party's shares (k_beaver32): a thread produces triple j of 16 rounds 64 apart, so each pass of
+// a wavefront stores 64 consecutive words of each output array; a block takes 1024 whole rounds.
+// Every party's (k_beaver32_all): a wavefront takes 256 consecutive triples. The field products are
+// exact 32 x 32 -> 64-bit multiplies folded by 2^31 = 1 (mod p); the shares of one party take the
+// product by its evaluation point 1..8 as a sum of 31-bit rotations, those of every party are running
+// sums; every value is kept in [0, p).
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -137,21 +139,104 @@ __global__ __launch_bounds__(64 * SPR) void k_beaver32(TripleArgs a) {
     const uint32_t lane = a.group == 32u ? (r & 31u) : r;
     const uint32_t bt = lane < 8u ? s_bt[a.group == 32u ? (r >> 5) - g0 : 0u][j] : 0u;
     const uint32_t ab = fmul(a0, b0);
-    if (a.party >= 0) {
-      const uint32_t x = a.eval[a.party];
-      // streaming stores: the outputs are written once and not read back by this kernel
-      __builtin_nontemporal_store(fadd(a0, fmul_small(ca, x)), a.a + k);
-      __builtin_nontemporal_store(fadd(b0, fmul_small(cb, x)), a.b + k);
-      __builtin_nontemporal_store(fadd(ab, fmul_small(bt, x)), a.c + k);
-    } else {
-      for (uint32_t p = 0; p < a.n; p++) {
-        const uint32_t x = a.eval[p];
-        const size_t o = (size_t)p * a.count + k;
-        __builtin_nontemporal_store(fadd(a0, fmul_small(ca, x)), a.a + o);
-        __builtin_nontemporal_store(fadd(b0, fmul_small(cb, x)), a.b + o);
-        __builtin_nontemporal_store(fadd(ab, fmul_small(bt, x)), a.c + o);
-      }
+    const uint32_t x = a.eval[a.party];
+    // streaming stores: the outputs are written once and not read back by this kernel
+    __builtin_nontemporal_store(fadd(a0, fmul_small(ca, x)), a.a + k);
+    __builtin_nontemporal_store(fadd(b0, fmul_small(cb, x)), a.b + k);
+    __builtin_nontemporal_store(fadd(ab, fmul_small(bt, x)), a.c + k);
+  }
+}
+
+// Every party's shares. 3 n output rows of count words, party p's starting at word p * count: with
+// one word per lane and store, rows that do not start on a 64-byte piece of HBM were written as
+// partial pieces (n = 5, 5 000 001 triples: 143 us; 5 000 000: 76 us). Here lane l of a wavefront
+// takes triples 4 l .. 4 l + 3 of 256 consecutive ones and stores 16 bytes per row; rows that start on
+// a piece are stored past the caches, the others through the L2, which joins the pieces that two
+// wavefronts share. Measured (us): 5 000 001 triples 72 (past the caches 83), 5 000 000 61 (through the
+// L2 64): 4.3 and 5.0 TB/s where a plain fill writes 6.8. Spans of 512 and 1024 triples, shifted to
+// whole pieces through LDS: 72-78 and 60-70.
+// bt_r as above, per wavefront: 8 lanes hash the first 8 rounds of each threadgroup of 32 rounds that
+// the span overlaps and reduce them, and every triple reads its group's sum across lanes.
+typedef uint32_t u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+constexpr uint32_t kAllBlock = 256, kSpan = 256;
+
+template <int SPR>
+__global__ __launch_bounds__(kAllBlock) void k_beaver32_all(TripleArgs a) {
+  constexpr uint32_t kGroups = (kSpan + SPR - 2) / SPR / 32 + 2;  // threadgroups of 32 rounds a span overlaps
+  constexpr uint32_t kPasses = (kGroups + 7) / 8;
+  const uint32_t lane = threadIdx.x & 63, last = a.num_rounds - 1u;
+  const uint32_t sp = blockIdx.x * (kAllBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t K0 = sp * kSpan, r0 = K0 / SPR, j0 = K0 - r0 * SPR;
+  if (K0 >= a.count) return;  // (uniform over the wavefront)
+  const uint32_t g0 = a.group == 32u ? r0 / 32u : 0u;  // (one group when num_rounds < 32)
+  uint32_t seedv[4], gseed[kPasses];
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) seedv[q] = a.seeds[min(r0 + (j0 + 4 * lane + q) / SPR, last)];
+#pragma unroll
+  for (uint32_t ps = 0; ps < kPasses; ps++)
+    gseed[ps] = a.seeds[min((g0 + 8 * ps + lane / 8) * a.group + (lane & 7), last)];
+  uint32_t gsum[kPasses][SPR];
+#pragma unroll
+  for (uint32_t ps = 0; ps < kPasses; ps++) {
+    const uint32_t i = lane & 7, r = (g0 + 8 * ps + lane / 8) * a.group + i;
+    const uint32_t h = i < a.n && i < a.group && r <= last ? chash32(gseed[ps], 3u * i) : 0u;
+#pragma unroll
+    for (int j = 0; j < SPR; j++) {
+      uint32_t v = fmul(a.him[j][i], h);
+      v = fadd(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));  // lane xor 1
+      v = fadd(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));  // lane xor 2
+      v = fadd(v, (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x1F | (4 << 10)));          // lane xor 4
+      gsum[ps][j] = v;
     }
+  }
+  uint32_t av[4], bv[4], cv[4], ca[4], cb[4], bt[4];
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) {
+    const uint32_t t = j0 + 4 * lane + q, dr = t / SPR, j = t - dr * SPR, r = r0 + dr;
+    const uint32_t hj = j == 0 ? 0u : j == 1 ? 2u * 0x9e3779b9u : 4u * 0x9e3779b9u;  // hmul[j] - hmul[0]
+    av[q] = chash32_m(seedv[q], a.hmul[0][0] + hj);
+    bv[q] = chash32_m(seedv[q], a.hmul[0][1] + hj);
+    ca[q] = chash32_m(seedv[q], a.hmul[0][2] + hj);
+    cb[q] = chash32_m(seedv[q], a.hmul[0][3] + hj);
+    cv[q] = fmul(av[q], bv[q]);
+    // lane r % group of threadgroup r / group (group = 32, or the one group of a short call)
+    const uint32_t gl = a.group == 32u ? (r & 31u) : r, gi = a.group == 32u ? (r >> 5) - g0 : 0u;
+    uint32_t b = 0u;
+#pragma unroll
+    for (uint32_t ps = 0; ps < kPasses; ps++)
+#pragma unroll
+      for (int jj = 0; jj < SPR; jj++) {
+        const uint32_t w = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(32u * (gi & 7u)), (int)gsum[ps][jj]);
+        b = gi / 8u == ps && j == (uint32_t)jj ? w : b;
+      }
+    bt[q] = gl < 8u ? b : 0u;
+  }
+  const uint32_t l = 4 * lane, left = a.count - K0;
+  auto put = [&](uint32_t *p, const uint32_t (&v)[4]) {
+    if (l + 4 <= left) {
+      const u32x4a4 w = {v[0], v[1], v[2], v[3]};
+      if (reinterpret_cast<uintptr_t>(p) & 63)  // (uniform)
+        *reinterpret_cast<u32x4a4 *>(p + l) = w;
+      else
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4a4 *>(p + l));
+    } else {
+#pragma unroll
+      for (uint32_t q = 0; q < 4; q++)
+        if (l + q < left) p[l + q] = v[q];
+    }
+  };
+  // the evaluation points are 1, 2, .. n: each party's shares are the one before's plus the slopes
+  size_t o = K0;
+  for (uint32_t p = 0; p < a.n; p++, o += a.count) {
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++) {
+      av[q] = fadd(av[q], ca[q]);
+      bv[q] = fadd(bv[q], cb[q]);
+      cv[q] = fadd(cv[q], bt[q]);
+    }
+    put(a.a + o, av);
+    put(a.b + o, bv);
+    put(a.c + o, cv);
   }
 }
 
@@ -199,6 +284,17 @@ int check_count(const beaver32_ctx *c, size_t count) {
   return MOE_OK;
 }
 
+// One party alone stays with k_beaver32: its 3 rows leave the hashes as the bound, and their sums over
+// a threadgroup cost least per block (20 M triples: 64 us against 87 us in spans).
+template <int SPR>
+void launch_spr(const TripleArgs &ta, hipStream_t s) {
+  if (ta.party < 0)
+    hipLaunchKernelGGL(k_beaver32_all<SPR>, dim3((ta.count + kSpan * (kAllBlock / 64) - 1) / (kSpan * (kAllBlock / 64))),
+                       dim3(kAllBlock), 0, s, ta);
+  else
+    hipLaunchKernelGGL(k_beaver32<SPR>, dim3((ta.num_rounds + kRounds - 1) / kRounds), dim3(64 * SPR), 0, s, ta);
+}
+
 int launch(beaver32_ctx *c, long party, size_t count, const uint32_t *seeds, uint32_t *a, uint32_t *b,
            uint32_t *cc, hipStream_t s) {
   if (!count) return MOE_OK;
@@ -224,11 +320,10 @@ int launch(beaver32_ctx *c, long party, size_t count, const uint32_t *seeds, uin
     ta.hmul[j][2] = base * 0x9e3779b9u;
     ta.hmul[j][3] = (base + 1u) * 0x9e3779b9u;
   }
-  const dim3 grid((unsigned)((ta.num_rounds + kRounds - 1) / kRounds));
   switch (c->spr) {
-    case 1: hipLaunchKernelGGL(k_beaver32<1>, grid, dim3(64), 0, s, ta); break;
-    case 2: hipLaunchKernelGGL(k_beaver32<2>, grid, dim3(128), 0, s, ta); break;
-    default: hipLaunchKernelGGL(k_beaver32<3>, grid, dim3(192), 0, s, ta); break;
+    case 1: launch_spr<1>(ta, s); break;
+    case 2: launch_spr<2>(ta, s); break;
+    default: launch_spr<3>(ta, s); break;
   }
   BV_HIP(hipGetLastError());
   return MOE_OK;

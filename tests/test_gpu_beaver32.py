@@ -62,3 +62,25 @@ def test_device_form_and_property(orc):
     with pytest.raises(MoeError, match="party"):
         g.generate_single_party(n, 10, seeds)
     g.close()
+
+
+@pytest.mark.parametrize("n,t", [(3, 1), (4, 1), (5, 1), (5, 2), (8, 3), (7, 3), (6, 2)])
+@pytest.mark.parametrize("count", [3, 31, 93, 255, 256, 257, 1024, 1027, 4093])
+def test_every_party_spans(orc, n, t, count):
+    """The wavefront spans of the all-party kernel: counts at the edges of 256 triples, fewer rounds
+    than one threadgroup, rows that start on and off a 64-byte piece (count a multiple of 16 or not,
+    a base pointer 4 bytes off), one to three triples per round; no word outside the rows written."""
+    g = GpuTripleGen32(n, t)
+    seeds = _seeds(count, g.spr, 700 + count)
+    want = orc.beaver32(n, t, count, seeds)
+    sd = DeviceBuffer.from_array(seeds)
+    for off in (0, 4):
+        outs = [DeviceBuffer.from_array(np.full(n * count + 8, 0xA5A5A5A5, np.uint32)) for _ in range(3)]
+        g.generate_device(-1, count, sd, *[o.ptr + off for o in outs])
+        g.synchronize()
+        for w, o, name in zip(want, outs, "abc"):
+            x = o.download(np.uint32, (n * count + 8,))
+            lead = off // 4
+            assert np.array_equal(x[lead:lead + n * count].reshape(n, count), w), f"{name} offset {off}"
+            assert (x[:lead] == 0xA5A5A5A5).all() and (x[lead + n * count:] == 0xA5A5A5A5).all()
+    g.close()
