@@ -237,11 +237,18 @@ __device__ __forceinline__ void router_compute(const RouterRegs<RNQ, RB> &R, con
   }
 }
 
+// The biases of the lane's 4 rows (gemv_epilogue's) of tile t of the record at rec (a raw matrix has none).
+template <int MODE>
+__device__ __forceinline__ float4 gemv_bias(const GemvArgs &a, const uint8_t *rec, int t, int lane) {
+  if (MODE == GEMV_RAW) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  return *reinterpret_cast<const float4 *>(rec + a.bias_off + 4 * (size_t)(t * 16 + (lane >> 4) * 4));
+}
+
 // Epilogue of one 16-row tile x 8-entry chunk. acc holds rows 4*(lane/16)+i of column
 // lane%16 (entry (lane%16)/2, term hi/lo); hi and lo columns are summed across lane pairs.
 template <int MODE>
 __device__ __forceinline__ void gemv_epilogue(const GemvArgs &a, const f32x4 &acc,
-                                              const uint8_t *rec, int beg, int c0, int nent,
+                                              const float4 &b, int beg, int c0, int nent,
                                               int t, int lane) {
   const int g = lane >> 4, j = lane & 15;
   float r[4];
@@ -252,10 +259,9 @@ __device__ __forceinline__ void gemv_epilogue(const GemvArgs &a, const f32x4 &ac
   const int ge = beg + el;
   const int r0 = t * 16 + g * 4;
   if (MODE == GEMV_GATE_UP) {
-    const float *bias = reinterpret_cast<const float *>(rec + a.bias_off);
     const int I = (int)a.d.rows / 2;
-    const float h0 = swiglu(r[0] + bias[r0], r[1] + bias[r0 + 1], a.limit);
-    const float h1 = swiglu(r[2] + bias[r0 + 2], r[3] + bias[r0 + 3], a.limit);
+    const float h0 = swiglu(r[0] + b.x, r[1] + b.y, a.limit);
+    const float h1 = swiglu(r[2] + b.z, r[3] + b.w, a.limit);
     uint16_t hi0, lo0, hi1, lo1;
     split_bf16(h0, hi0, lo0);
     split_bf16(h1, hi1, lo1);
@@ -264,13 +270,12 @@ __device__ __forceinline__ void gemv_epilogue(const GemvArgs &a, const f32x4 &ac
     *reinterpret_cast<uint32_t *>(hs + ii) = (uint32_t)hi0 | ((uint32_t)hi1 << 16);
     *reinterpret_cast<uint32_t *>(hs + I + ii) = (uint32_t)lo0 | ((uint32_t)lo1 << 16);
   } else if (MODE == GEMV_DOWN) {
-    const float *bias = reinterpret_cast<const float *>(rec + a.bias_off);
     float *o = reinterpret_cast<float *>(a.out) + (size_t)ge * a.d.rows + r0;
     float4 v4;
-    v4.x = canon_nan(rclamp(r[0] + bias[r0], -65504.0f, 65504.0f));
-    v4.y = canon_nan(rclamp(r[1] + bias[r0 + 1], -65504.0f, 65504.0f));
-    v4.z = canon_nan(rclamp(r[2] + bias[r0 + 2], -65504.0f, 65504.0f));
-    v4.w = canon_nan(rclamp(r[3] + bias[r0 + 3], -65504.0f, 65504.0f));
+    v4.x = canon_nan(rclamp(r[0] + b.x, -65504.0f, 65504.0f));
+    v4.y = canon_nan(rclamp(r[1] + b.y, -65504.0f, 65504.0f));
+    v4.z = canon_nan(rclamp(r[2] + b.z, -65504.0f, 65504.0f));
+    v4.w = canon_nan(rclamp(r[3] + b.w, -65504.0f, 65504.0f));
     *reinterpret_cast<float4 *>(o) = v4;
   } else {
     float *o = reinterpret_cast<float *>(a.out) + (size_t)ge * a.d.rows + r0;

@@ -62,7 +62,7 @@ struct GemvArgs {
   size_t mat_off;          // packed matrix offset inside a record
   size_t bias_off;         // f32 bias offset inside a record (ignored for GEMV_RAW)
   PackDims d;              // matrix dimensions
-  const int32_t *n_active; // device scalar: active experts this call
+  const int32_t *n_active; // device scalar: active experts this call (NULL: one entry of the record at base)
   const int32_t *active_ids, *active_off;
   const int32_t *entry_src;  // B row of each entry (NULL: the entry itself)
   const uint16_t *bsrc;      // [rows_b, 2, K] bf16 hi/lo operands, K = d.nb * 32
