@@ -108,7 +108,12 @@ __host__ __device__ constexpr int route_hp(int H) { return ((H + 63) / 64 + 7) /
 // With xrec the block also writes its tokens' grouped-GEMM records; with bucket_ticket the last
 // block to finish groups every entry by expert (bucket_block) in its free x staging area.
 // NT: the records' terms.
-template <int KI, int TB, int NT>
+// NORM (the block forward): the staged rows are RMS-normalised first: one wavefront per token sums
+// the squares of the staged row in rms_inv_wave's order, and every thread scales the values it
+// staged, (x r) gamma, as k_rmsnorm does: the same bits, without that kernel's launch and its pass
+// over x (7 tokens of 2880: k_rmsnorm 7.2 us + k_route 7.1 -> 8.6 us traced; 333 of 2048: 6.2 + 16.0
+// -> 19.2).
+template <int KI, int TB, int NT, bool NORM>
 __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   __shared__ float s_logit[TB][kMaxExperts];
   __shared__ float s_p[kMaxExperts];
@@ -117,6 +122,7 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   __shared__ int s_sel[TB];
   __shared__ int s_last;
   __shared__ int s_cnt[kMaxExperts];  // the grouping's per-expert counts of the block's entries
+  __shared__ float s_r[NORM ? TB : 1];  // the tokens' 1 / rms
   const int t0 = blockIdx.x * TB;
   const int nt = min(TB, a.T - t0);
   const int lane = threadIdx.x & 63;
@@ -156,12 +162,61 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
         const int k = (int)threadIdx.x + q * kRouteThreads;
         xv[tb][q] = tb < nt && k < H ? a.x[(size_t)(t0 + tb) * H + k] : 0.0f;
       }
+    if constexpr (NORM) {
+      float gm[kPer];
+#pragma unroll
+      for (int q = 0; q < kPer; q++) {
+        const int k = (int)threadIdx.x + q * kRouteThreads;
+        gm[q] = k < H ? a.gamma[k] : 0.0f;
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++)
+          if (tb < nt && k < Hp) s_x[tb * Hp + k] = xv[tb][q];
+      }
+      __syncthreads();
+      if (wv < nt) {
+        float sq[KI * 8], p = 0.0f;  // (zeros from H to Hp add nothing)
+#pragma unroll
+        for (int i = 0; i < KI * 8; i++) {
+          const float v1 = s_x[wv * Hp + lane + 64 * i];
+          sq[i] = v1 * v1;
+        }
+#pragma unroll
+        for (int i = 0; i < KI * 8; i++) p = p + sq[i];
+        const float r = 1.0f / sqrtf(wave_sum_xor(p) / (float)H + a.eps);
+        if (lane == 0) s_r[wv] = r;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int tb = 0; tb < TB; tb++) {
+        const float r = s_r[tb < nt ? tb : 0];
+#pragma unroll
+        for (int q = 0; q < kPer; q++) {
+          const float vr = xv[tb][q] * r;
+          xv[tb][q] = vr * gm[q];
+        }
+      }
+    }
 #pragma unroll
     for (int tb = 0; tb < TB; tb++)
 #pragma unroll
       for (int q = 0; q < kPer; q++) {
         const int k = (int)threadIdx.x + q * kRouteThreads;
-        if (tb < nt && k < Hp) stage(tb, k, xv[tb][q]);
+        // (with a norm the rows' padding is zero already, and must not become inf * 0)
+        if (tb < nt && k < (NORM ? H : Hp)) stage(tb, k, xv[tb][q]);
+      }
+  } else if constexpr (NORM) {
+    for (int tb = 0; tb < nt; tb++)
+      for (int k = threadIdx.x; k < Hp; k += kRouteThreads) s_x[tb * Hp + k] = k < H ? a.x[(size_t)(t0 + tb) * H + k] : 0.0f;
+    __syncthreads();
+    if (wv < nt) {
+      const float r = rms_inv_wave(s_x + wv * Hp, H, a.eps, lane);
+      if (lane == 0) s_r[wv] = r;
+    }
+    __syncthreads();
+    for (int tb = 0; tb < nt; tb++)
+      for (int k = threadIdx.x; k < H; k += kRouteThreads) {
+        const float vr = s_x[tb * Hp + k] * s_r[tb];
+        stage(tb, k, vr * a.gamma[k]);
       }
   } else {
     for (int tb = 0; tb < nt; tb++)
@@ -415,15 +470,20 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   }
 }
 
-template <int KI, int TB, int NT>
-static hipError_t launch_route_tb(const RouteArgs &a, size_t hp, hipStream_t s) {
+template <int KI, int TB, int NT, bool NORM>
+static hipError_t launch_route_norm(const RouteArgs &a, size_t hp, hipStream_t s) {
   if (TB * hp > 65536) {  // more than the default 64 KB of dynamic LDS
     static DynLdsOnce once;
-    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, TB, NT>), TB * hp);
+    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, TB, NT, NORM>), TB * hp);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_route<KI, TB, NT>), dim3((unsigned)((a.T + TB - 1) / TB)), dim3(kRouteThreads), TB * hp, s, a);
+  hipLaunchKernelGGL((k_route<KI, TB, NT, NORM>), dim3((unsigned)((a.T + TB - 1) / TB)), dim3(kRouteThreads), TB * hp, s, a);
   return hipGetLastError();
+}
+
+template <int KI, int TB, int NT>
+static hipError_t launch_route_tb(const RouteArgs &a, size_t hp, hipStream_t s) {
+  return a.gamma ? launch_route_norm<KI, TB, NT, true>(a, hp, s) : launch_route_norm<KI, TB, NT, false>(a, hp, s);
 }
 
 template <int KI>
@@ -730,76 +790,76 @@ hipError_t launch_gemv(GemvMode mode, const GemvArgs &a, hipStream_t s) {
 
 // y[t, d] = sum over slots s (rank order) of w[t, s] * o[pos[t, s], d], accumulated from 0
 // with separate rounding of each product and sum (session.rs:975-980). skip_nonfinite drops
-// non-finite o elements (moe_dispatch.rs:598-601).
-__global__ __launch_bounds__(256) void k_combine(const float *o, const int32_t *pos,
-                                                 const float *w, int T, int k, int H,
-                                                 int skip_nonfinite, float *y) {
+// non-finite o elements (moe_dispatch.rs:598-601). With resid the row's residual is added last
+// (session.rs:982-994: hidden + moe_out; resid may be 4-byte aligned), in place of a launch of
+// k_add_rows (about 4 us at a few tokens, all launch). K > 0: k = K, every slot's row load is issued
+// before the first product; K = 0: any k, one round trip per slot.
+template <int K>
+__global__ __launch_bounds__(256) void k_combine(const float *o, const int32_t *pos, const float *w, int T, int k,
+                                                 int H, int skip_nonfinite, const float *resid, float *y) {
   const int h4 = H / 4;
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (size_t)T * h4) return;
   const int t = (int)(i / h4), d4 = (int)(i % h4);
+  float xr[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (resid) {
+    const float *r = resid + (size_t)t * H + 4 * d4;
+    if (reinterpret_cast<uintptr_t>(resid) & 15) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) xr[c] = r[c];
+    } else {
+      const float4 v = *reinterpret_cast<const float4 *>(r);
+      xr[0] = v.x;
+      xr[1] = v.y;
+      xr[2] = v.z;
+      xr[3] = v.w;
+    }
+  }
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s = 0; s < k; s++) {
-    const int p = pos[(size_t)t * k + s];
-    if (p < 0) continue;
-    const float ws = w[(size_t)t * k + s];
-    const float4 v = reinterpret_cast<const float4 *>(o + (size_t)p * H)[d4];
+  auto add = [&](const float4 &v, float ws) {
     const float vv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       if (skip_nonfinite && !isfinite(vv[c])) continue;
       acc[c] = acc[c] + ws * vv[c];
     }
-  }
-  reinterpret_cast<float4 *>(y + (size_t)t * H)[d4] =
-      make_float4(canon_nan(acc[0]), canon_nan(acc[1]), canon_nan(acc[2]), canon_nan(acc[3]));
-}
-
-// k_combine for a fixed k: every slot's row load is issued before the first product, instead of
-// one round trip per slot (the same products and sums in the same order).
-template <int K>
-__global__ __launch_bounds__(256) void k_combine_k(const float *o, const int32_t *pos,
-                                                   const float *w, int T, int H, int skip_nonfinite,
-                                                   float *y) {
-  const int h4 = H / 4;
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)T * h4) return;
-  const int t = (int)(i / h4), d4 = (int)(i % h4);
-  int p[K];
-  float ws[K];
-  float4 v[K];
+  };
+  if constexpr (K > 0) {
+    int p[K];
+    float ws[K];
+    float4 v[K];
 #pragma unroll
-  for (int s = 0; s < K; s++) {
-    p[s] = pos[(size_t)t * K + s];
-    ws[s] = w[(size_t)t * K + s];
-  }
-#pragma unroll
-  for (int s = 0; s < K; s++)  // a dropped slot (p < 0) reads row 0 and is not used
-    v[s] = reinterpret_cast<const float4 *>(o + (size_t)(p[s] < 0 ? 0 : p[s]) * H)[d4];
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < K; s++) {
-    if (p[s] < 0) continue;
-    const float vv[4] = {v[s].x, v[s].y, v[s].z, v[s].w};
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      if (skip_nonfinite && !isfinite(vv[c])) continue;
-      acc[c] = acc[c] + ws[s] * vv[c];
+    for (int s = 0; s < K; s++) {
+      p[s] = pos[(size_t)t * K + s];
+      ws[s] = w[(size_t)t * K + s];
     }
+#pragma unroll
+    for (int s = 0; s < K; s++)  // a dropped slot (p < 0) reads row 0 and is not used
+      v[s] = reinterpret_cast<const float4 *>(o + (size_t)(p[s] < 0 ? 0 : p[s]) * H)[d4];
+#pragma unroll
+    for (int s = 0; s < K; s++)
+      if (p[s] >= 0) add(v[s], ws[s]);
+  } else {
+    for (int s = 0; s < k; s++) {
+      const int p = pos[(size_t)t * k + s];
+      if (p >= 0) add(reinterpret_cast<const float4 *>(o + (size_t)p * H)[d4], w[(size_t)t * k + s]);
+    }
+  }
+  if (resid) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = xr[c] + acc[c];
   }
   reinterpret_cast<float4 *>(y + (size_t)t * H)[d4] =
       make_float4(canon_nan(acc[0]), canon_nan(acc[1]), canon_nan(acc[2]), canon_nan(acc[3]));
 }
 
 hipError_t launch_combine(const float *o, const int32_t *pos, const float *w, int T, int k, int H,
-                          int skip_nonfinite, float *y, hipStream_t s) {
+                          int skip_nonfinite, const float *resid, float *y, hipStream_t s) {
   if (H % 4 || T < 1 || k < 1) return hipErrorInvalidValue;
   const size_t n = (size_t)T * (H / 4);
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-  if (k == 4)
-    hipLaunchKernelGGL(k_combine_k<4>, grid, block, 0, s, o, pos, w, T, H, skip_nonfinite, y);
-  else
-    hipLaunchKernelGGL(k_combine, grid, block, 0, s, o, pos, w, T, k, H, skip_nonfinite, y);
+  auto kern = k == 1 ? k_combine<1> : k == 2 ? k_combine<2> : k == 4 ? k_combine<4> : k_combine<0>;
+  hipLaunchKernelGGL(kern, grid, block, 0, s, o, pos, w, T, k, H, skip_nonfinite, resid, y);
   return hipGetLastError();
 }
 

@@ -40,6 +40,8 @@ struct RouteArgs {
   const uint16_t *w;     // load-major router: [E][KIp/8][64 lanes][8] bf16 bits (router_dot)
   const float *bias;     // [E]
   const float *x;        // [T, H]
+  const float *gamma;    // non-null: the rows are RMS-normalised with it first (the block forward)
+  float eps;
   int T, E, H, k;
   int adaptive, min_k;
   float top1_min, margin_min, top2_mass;
@@ -209,7 +211,7 @@ hipError_t launch_bucket(const int32_t *idx, int T, int k, int E, int32_t *n_act
                          int32_t *pos, hipStream_t s);
 hipError_t launch_gemv(GemvMode mode, const GemvArgs &a, hipStream_t s);
 hipError_t launch_combine(const float *o, const int32_t *pos, const float *w, int T, int k, int H,
-                          int skip_nonfinite, float *y, hipStream_t s);
+                          int skip_nonfinite, const float *resid, float *y, hipStream_t s);
 hipError_t launch_split(const float *x, size_t n_rows, size_t K, uint16_t *xsplit, hipStream_t s);
 hipError_t launch_dequant_hf(const uint8_t *blocks, const uint8_t *scales, size_t rows,
                              size_t cols, float *out, hipStream_t s);

@@ -102,7 +102,7 @@ struct Layer {
 
 // Per-call device scratch, carved from one allocation.
 struct Work {
-  float *x, *y, *logits, *wts, *o, *xn;  // xn: normalised rows of the block forward
+  float *x, *y, *logits, *wts, *o, *xn;  // xn: the normalised row of a single token's block forward
   uint16_t *xsplit, *hsplit;
   uint8_t *xrec, *hrec;  // grouped GEMM activation records: tokens, entries (padding zero)
   int32_t *idx, *n_active, *active_ids, *active_off, *entry_src, *pos;
@@ -236,7 +236,7 @@ size_t router_bytes(size_t H, size_t E) { return E * 64 * router_kip(H) * 2; }
 
 // Lays out the per-call workspace of T tokens, top-k k and E experts at `b` (nullptr: sizes
 // only) and returns its bytes. host_io adds the staging rows of host-pointer calls (x, y) and
-// the normalised rows of the unfused block forward (xn).
+// the normalised row of the single token's unfused block forward (xn).
 // what: with WORK_FINE only the operands of the four-term small-batch GEMM, with WORK_COARSE those
 // of the other paths.
 size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size_t I, bool host_io, WorkFor what) {
@@ -252,7 +252,7 @@ size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size
   };
   w.x = (float *)take(host_io ? T * H * 4 : 0);
   w.y = (float *)take(host_io ? T * H * 4 : 0);
-  w.xn = (float *)take(host_io ? T * H * 4 : 0);
+  w.xn = (float *)take(host_io ? H * 4 : 0);
   w.logits = (float *)take(T * E * 4);
   w.wts = (float *)take(N * 4);
   w.o = (float *)take(N * H * 4);
@@ -487,8 +487,9 @@ bool takes_fine(const moe_ctx *c, const Layer &Ly, size_t T, size_t k, const flo
          gemm_fine_fits(gemm_args(c, Ly, T, k), c->L.dn);
 }
 
-// norm: the block forward (RMSNorm of x before, x + result after); the one-launch decode fuses
-// both, the other paths run k_rmsnorm into the workspace first and k_add_rows last.
+// norm: the block forward (RMSNorm of x before, x + result after). The one-launch decode fuses
+// both; the batch path normalises in its router and adds the residual in its combine; the two-launch
+// decode runs k_rmsnorm into the workspace first and k_add_rows last.
 // w: the workspace, sized for (T, k, E) by the caller (ensure_work, or the scratch array of the
 // allocation-free entry point).
 int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size_t T, size_t k,
@@ -503,10 +504,14 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   if (!x || !y) return fail(MOE_ERR_INVALID, "null x or y");
   RETURN_IF(check_tokens(c->layers[layer].n_experts, T, k));
   if (norm && !Ly.has_norm) return fail(MOE_ERR_STATE, "layer %zu has no RMSNorm weight", layer);
-  const float *resid = nullptr;  // x for the residual add of the unfused paths
+  const float *resid = nullptr;  // x for the residual add of the paths that end with one
+  bool route_norm = false;       // the router normalises
   if (norm) {
-    const bool fused = T == 1 && c->decode_mode == 2;
-    if (!fused || (reinterpret_cast<uintptr_t>(x) & 15)) {
+    if (T > 1 || c->decode_mode == 0) {
+      route_norm = true;
+      resid = x;
+      norm = false;
+    } else if (c->decode_mode != 2 || (reinterpret_cast<uintptr_t>(x) & 15)) {
       RETURN_IF(timed(c, K_NORM, s, [&] {
         return launch_rmsnorm(x, T, c->H, (const float *)Ly.norm.p, Ly.eps, w.xn, s);
       }));
@@ -577,6 +582,10 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   ra.w = (const uint16_t *)Ly.router.p;
   ra.bias = (const float *)((const char *)Ly.router.p + al(router_bytes(c->H, E)));
   ra.x = x;
+  if (route_norm) {
+    ra.gamma = (const float *)Ly.norm.p;
+    ra.eps = Ly.eps;
+  }
   ra.T = (int)T;
   ra.E = (int)E;
   ra.H = (int)c->H;
@@ -592,10 +601,12 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   // the grouped GEMM (16- to 64-entry column tiles) pays off once experts average a few
   // entries; smaller batches stream each weight tile through the GEMV kernels, which read the
   // bf16 hi + lo split of x that the router writes
-  const bool fine = w.hfine && takes_fine(c, Ly, T, k, x);
+  // (unaligned x rows take the GEMV path, unless the router writes normalised ones)
+  const float *rows = route_norm ? w.xn : x;
+  const bool fine = w.hfine && takes_fine(c, Ly, T, k, rows);
   const bool use_gemm = fine || (c->batch_gemm && T > 1 && (c->batch_gemm == 2 || T * k >= 4 * E) &&
                                  c->L.gu.ns <= (uint32_t)kGemmNs && c->L.dn.ns <= (uint32_t)kGemmNs &&
-                                 (reinterpret_cast<uintptr_t>(x) & 15) == 0);
+                                 (reinterpret_cast<uintptr_t>(rows) & 15) == 0);
   ra.xsplit = use_gemm ? nullptr : w.xsplit;
   ra.xrec = fine ? w.xfine : use_gemm ? w.xrec : nullptr;  // the router writes the GEMM's activation records
   ra.rec_terms = fine ? kFineTerms : c->act_quant ? 1 : kGemmTerms;
@@ -666,9 +677,8 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
     RETURN_IF(run_experts(c, w, (const uint8_t *)Ly.experts.p, max_active, (int)std::min(T, (size_t)1 << 30), s));
   }
   RETURN_IF(timed(c, K_COMBINE, s, [&] {
-    return launch_combine(w.o, w.pos, w.wts, (int)T, (int)k, (int)c->H, 0, y, s);
+    return launch_combine(w.o, w.pos, w.wts, (int)T, (int)k, (int)c->H, 0, resid, y, s);
   }));
-  if (resid) RETURN_IF(timed(c, K_NORM, s, [&] { return launch_add_rows(y, resid, T * c->H, s); }));
   return MOE_OK;
 }
 
@@ -933,7 +943,7 @@ int moe_dispatch_experts_batched(moe_ctx *c, const float *input, size_t n,
   for (size_t i = 0; i < n; i++) wts[i] = ex[i].weight;
   HIP_TRY(hipMemcpyAsync(c->w.wts, wts.data(), n * 4, hipMemcpyHostToDevice, c->stream));
   RETURN_IF(run_experts(c, c->w, base, (int)n, 1, c->stream));
-  HIP_TRY(launch_combine(c->w.o, c->w.pos, c->w.wts, 1, (int)n, (int)c->H, 1, c->w.y, c->stream));
+  HIP_TRY(launch_combine(c->w.o, c->w.pos, c->w.wts, 1, (int)n, (int)c->H, 1, nullptr, c->w.y, c->stream));
   HIP_TRY(hipMemcpyAsync(output, c->w.y, c->H * 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   return MOE_OK;

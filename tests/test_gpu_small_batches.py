@@ -131,3 +131,28 @@ def test_small_batch_adaptive_unaligned_and_replayed(orc):
             check(lib().moe_graph_destroy(g))
     finally:
         d.close()
+
+
+# H: a router of one and of two loads per lane, the runtime chain (2048), padding (H < 64 NQ); T: the
+# streamed forms, the 8-token router blocks with a partial one; k: each unrolled combine and the loop
+@pytest.mark.parametrize("H,E,k,T", [(96, 8, 1, 5), (544, 8, 2, 40), (2048, 16, 3, 9), (2880, 8, 4, 2053), (1024, 8, 8, 33)])
+def test_block_norm_in_router_and_residual_in_combine(orc, H, E, k, T):
+    """The batch's block forward gives the same bits as x + layer_forward(oracle RMSNorm(x)), also
+    for rows of zeros and of huge values and for x at a 4-byte alignment."""
+    L = syn.make_layer(H, 96, E, seed=660 + H, scale_lo=117, scale_hi=121, router_sigma=0.1)
+    rng = np.random.default_rng(661)
+    gamma = (1 + 0.2 * rng.standard_normal(H)).astype(np.float32)
+    d = GpuMoeDispatcher(H, 96, 7.0)
+    try:
+        d.preload_layer(0, L)
+        d.preload_norm(0, gamma, 1e-5)
+        x = (3 * syn.hidden(T, H, seed=662)).astype(np.float32)
+        x[1], x[2] = 0.0, 1e15 * x[2]
+        ref = (x + d.layer_forward(0, orc.rms_norm(x, gamma, 1e-5), k)).astype(np.float32)
+        assert np.array_equal(d.block_forward(0, x, k), ref)
+        flat, out = DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x.ravel()])), DeviceBuffer(x.nbytes)
+        check(lib().moe_block_forward_device(d.ctx, 0, ctypes.c_void_p(flat.ptr + 4), T, k, ctypes.c_void_p(out.ptr), None))
+        d.synchronize()
+        assert np.array_equal(out.download(np.float32, x.shape), ref)
+    finally:
+        d.close()
