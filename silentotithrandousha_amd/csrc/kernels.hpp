@@ -204,6 +204,10 @@ hipError_t launch_decode_gate_up(const DecodeArgs &a, hipStream_t s);
 hipError_t launch_decode_down(const DecodeArgs &a, hipStream_t s);
 
 hipError_t launch_route(const RouteArgs &a, hipStream_t s);
+// The router of larger batches on the f32 MFMA (route_wide.hip); group: also the grouping by expert
+// (in a second kernel). route_wide_fits: whether it takes these arguments.
+bool route_wide_fits(const RouteArgs &a);
+hipError_t launch_route_wide(RouteArgs a, bool group, hipStream_t s);
 // Whether k_route's x staging (one token) holds bucket_block's LDS for E experts.
 bool route_bucket_fits(int H, int E);
 hipError_t launch_bucket(const int32_t *idx, int T, int k, int E, int32_t *n_active,

@@ -650,12 +650,13 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
     gu.w_entry_src = w.entry_src;
     gu.w_pos = w.pos;
   }
-  const bool fuse_bucket = T > 1 && !local_group && route_bucket_fits((int)c->H, (int)E);
-  ra.bucket_ticket = fuse_bucket ? (uint32_t *)c->route_ticket.p : nullptr;
   ra.blk_count = w.blk_count;
   ra.rank = w.rank;
-  RETURN_IF(timed(c, K_ROUTE, s, [&] { return launch_route(ra, s); }));
-  if (T > 1 && !fuse_bucket && !local_group)
+  const bool wide_route = route_wide_fits(ra);
+  const bool fuse_bucket = !wide_route && T > 1 && !local_group && route_bucket_fits((int)c->H, (int)E);
+  ra.bucket_ticket = fuse_bucket ? (uint32_t *)c->route_ticket.p : nullptr;
+  RETURN_IF(timed(c, K_ROUTE, s, [&] { return wide_route ? launch_route_wide(ra, !local_group, s) : launch_route(ra, s); }));
+  if (!wide_route && T > 1 && !fuse_bucket && !local_group)
     RETURN_IF(timed(c, K_BUCKET, s, [&] {
       return launch_bucket(w.idx, (int)T, (int)k, (int)E, w.n_active, w.active_ids,
                            w.active_off, w.entry_src, w.pos, s);
@@ -1048,7 +1049,7 @@ int moe_router_topk(moe_ctx *c, size_t layer, const float *x, size_t T, size_t k
   ra.wts = c->w.wts;
   ra.xsplit = nullptr;
   ra.fuse_bucket = 0;
-  HIP_TRY(launch_route(ra, c->stream));
+  HIP_TRY(route_wide_fits(ra) ? launch_route_wide(ra, false, c->stream) : launch_route(ra, c->stream));
   HIP_TRY(hipMemcpyAsync(idx, c->w.idx, T * k * 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipMemcpyAsync(weights, c->w.wts, T * k * 4, hipMemcpyDeviceToHost, c->stream));
   if (logits)
