@@ -121,10 +121,11 @@ static_assert(kTerms == 4, "h record piece = 4 terms x 8 bytes");
 // policy (sc1: the h records are written by other blocks with agent-scope stores), written as
 // inline assembly so that the compiler's wait tracking does not see it (with the builtin it makes
 // every later LDS read wait for all DMAs in flight); the caller waits with counted vmcnt. Every
-// LDS-DMA of this kernel goes through here, so the compiler keeps no value of its own in m0.
+// LDS-DMA of this kernel goes through here, so the compiler keeps no value of its own in m0. (The
+// s_nop: one wait state between the write of m0 and the load.)
 __device__ __forceinline__ void lds_dma16_sc1(const void *g, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off sc1" ::"v"(g), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off sc1" ::"v"(g), "s"(la) : "memory", "m0");
 }
 
 // The down sweep of a loaded down tile against its slot's h record: the record (tile-major, 512

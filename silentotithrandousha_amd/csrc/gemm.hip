@@ -37,21 +37,23 @@ namespace moe {
 // lds + l * size (lds uniform over the wavefront). Written as inline assembly so that the compiler does not see these LDS writes:
 // it would otherwise make later LDS reads wait for every DMA in flight (it cannot always tell
 // the ring slots apart). The kernel orders them itself: vmcnt waits counted per step, then a
-// barrier, with compiler fences around it.
+// barrier, with compiler fences around it. The s_nop is the wait state that the load needs after the
+// write of m0; the forms with a base in SGPRs get it, and a base that no VALU instruction has just
+// written, by the move through vcc (stream.hpp).
 __device__ __forceinline__ void lds_dma16(const void *g, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory", "m0");
 }
 // The same with the non-temporal cache policy: for weight chunks read once per launch (the small
 // blocks of batches of a few entries per expert; measured at 64 tokens: down 37.5 -> 36.0 us; where
 // column tiles of one expert re-read the chunks, at prefill, it cost 4 %).
 __device__ __forceinline__ void lds_dma16_nt(const void *g, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(la) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_dma4(const void *g, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(la) : "memory", "m0");
 }
 
 // The LDS byte address of p (a pointer into a __shared__ object).
@@ -61,18 +63,21 @@ __device__ __forceinline__ uint32_t lds_addr(const void *p) {
 // LDS-DMA of 16 bytes per lane to the LDS byte address la (wavefront-uniform), from sbase + voff.
 __device__ __forceinline__ void lds_dma16_sa(uint32_t voff, const void *sbase, uint32_t la) {
   la = __builtin_amdgcn_readfirstlane(la);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 
 // The same with a wavefront-uniform 64-bit base in SGPRs and a 32-bit per-lane offset
 // (global address = sbase + voff): one VGPR per lane instead of a 64-bit pointer.
 __device__ __forceinline__ void lds_dma16_s(uint32_t voff, const void *sbase, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 __device__ __forceinline__ void lds_dma4_s(uint32_t voff, const void *sbase, const void *lds) {
   const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)lds);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dword %0, vcc" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 
 // Block shape: WR x WC wavefronts; wavefront (wr, wc) owns RT tiles of 16 weight rows (row

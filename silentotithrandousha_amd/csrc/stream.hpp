@@ -30,20 +30,28 @@ __device__ __forceinline__ void str_st1(void *p, uint32_t v) {
 
 // LDS-DMA of 16 bytes per lane from sbase + voff (wavefront-uniform base, 32-bit lane offset) to
 // LDS byte address la + 16 l. Inline assembly, so that the compiler does not make later LDS reads
-// wait for it; the kernel counts its own DMAs with vm_wait.
+// wait for it; the kernel counts its own DMAs with vm_wait. The base goes through vcc by a scalar
+// move: the compiler's wait states do not reach into assembly, and it may have written the base just
+// before by v_readlane (a spilled SGPR), a VALU write that a vector memory instruction may read only
+// 5 wait states later (884 of these loads read theirs after 1 to 4: a load from a stale address);
+// the move is also the wait state that the load needs after the write of m0. Layers unchanged by it
+// within the runs' spread.
 __device__ __forceinline__ void str_dma16(uint32_t voff, const void *sbase, uint32_t la) {
   la = __builtin_amdgcn_readfirstlane(la);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 // The same with the non-temporal cache policy (weights read once per launch).
 __device__ __forceinline__ void str_dma16_nt(uint32_t voff, const void *sbase, uint32_t la) {
   la = __builtin_amdgcn_readfirstlane(la);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc nt" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 // LDS-DMA of 4 bytes per lane (lane l's bytes land at la + 4 l).
 __device__ __forceinline__ void str_dma4(uint32_t voff, const void *sbase, uint32_t la) {
   la = __builtin_amdgcn_readfirstlane(la);
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(la) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 vcc, %1\n\tglobal_load_lds_dword %0, vcc" ::"v"(voff), "s"(sbase), "s"(la)
+               : "memory", "m0", "vcc");
 }
 __device__ __forceinline__ uint32_t str_lds(const void *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p;
