@@ -78,7 +78,7 @@ int moe_set_adaptive_topk(moe_ctx *ctx, int enabled, size_t min_k, float top1_mi
  * moe_layer_forward return MOE_ERR_HIP (which clears the condition).
  * MOE_OPT_BATCH_GEMM: batches (n_tokens > 1) run through the grouped GEMM on the block-scaled
  * MFMA when 1 (default): activations as 3 fp6 terms, exact to 2^-13 of a block's maximum, once
- * experts average at least 4 entries, and as 4 terms, exact to 2^-18, below that (the streamed
+ * experts average at least 4 entries, and as 6 terms, exact to 2^-28, below that (the streamed
  * form of code 12 with 8-entry chunks; MOE_OPT_GEMM_SHAPE and MOE_OPT_ACT_QUANT do not apply to
  * it). 2: always the 3-term form. 0, and batches that the grouped GEMM does not take (K above
  * 3072, x not 16-byte aligned, fewer than 96 rows): the per-tile GEMV kernels (bf16 hi+lo

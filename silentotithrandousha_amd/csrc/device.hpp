@@ -868,7 +868,8 @@ typedef uint32_t u32x6v __attribute__((ext_vector_type(6)));
 // [1/2, 1). Several terms: 2^(E - 2 - 5t) (term 0 holds the block in [-4, 4), so its residual
 // never saturates; each later term removes 5 more bits). One term (the quantized mode): the OCP
 // MX rule, 2^(floor(log2 m) - 2) = 2^(E - 3), the block maximum in [4, 8) (values past 7.5
-// saturate). Stops at 2^-126 (a normal f32) for blocks below about 2^-120.
+// saturate). Stops at 2^-126 (a normal f32): the last of NT terms for blocks below
+// 2^(5 NT - 129), whose values then keep 2^-130 absolute.
 template <int NT>
 __device__ __forceinline__ int split_scale_exp(int E, int t) {
   return max(NT == 1 ? E - 3 : E - 2 - 5 * t, -126);
@@ -950,27 +951,55 @@ __device__ __forceinline__ void split32_fp6(const float (&x)[32], float m, bool 
   }
 }
 
-// Block blk (values 32 blk .. 32 blk + 31, in v; 0 <= blk < 4 kGemmNs) of a row into the row's
-// GemmRecT<NT> record r: one lane per block (split32_fp6): the NT terms' codes and scale bytes.
-template <int NT>
-__device__ __forceinline__ void rec_split_block(const float (&v)[32], int blk, uint8_t *r) {
-  using R = GemmRecT<NT>;
+// split32_fp6 with each term's codes and scale byte handed to emit(t, codes, scale) as they are made:
+// six terms held until the last would not leave the streamed GEMM's epilogue its registers.
+template <int NT, typename F>
+__device__ __forceinline__ void split32_fp6_each(const float (&x)[32], F &&emit) {
   float m = 0.0f;
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < 32; i++) {
-    m = fmaxf(m, fabsf(v[i]));
-    bad = bad || !isfinite(v[i]);
+    m = fmaxf(m, fabsf(x[i]));
+    bad = bad || !isfinite(x[i]);
   }
-  uint32_t d[NT][6], sb;
-  split32_fp6<NT>(v, m, bad, d, sb);
-  const int st = blk >> 2, i = blk & 3;
+  int E = 0;
+  if (m > 0.0f && isfinite(m)) frexpf(m, &E);
+  f32x16v a, b;  // the residual's values 2 i and 2 i + 1
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    a[i] = bad ? 0.0f : x[2 * i];
+    b[i] = bad ? 0.0f : x[2 * i + 1];
+  }
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    *reinterpret_cast<uint4 *>(r + R::dword(st, t, i, 0)) = make_uint4(d[t][0], d[t][1], d[t][2], d[t][3]);
-    *reinterpret_cast<uint2 *>(r + R::dword(st, t, i, 4)) = make_uint2(d[t][4], d[t][5]);
-    r[R::scale(st, t) + i] = (uint8_t)(sb >> (8 * t));
+    const int se = split_scale_exp<NT>(E, t);
+    const float sc = __builtin_amdgcn_ldexpf(1.0f, se);
+    u32x6v c;
+    asm volatile("v_cvt_scalef32_2xpk16_fp6_f32 %0, %1, %2, %3" : "=&v"(c) : "v"(a), "v"(b), "v"(sc));
+    emit(t, c, bad ? 0xFFu : (uint32_t)(se + 127));
+    if (t + 1 < NT) {  // the residual feeds the next term (the last term needs none)
+      f32x32v q;
+      asm volatile("v_cvt_scalef32_pk32_f32_fp6 %0, %1, %2" : "=&v"(q) : "v"(c), "v"(sc));
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        a[i] = a[i] - q[2 * i];
+        b[i] = b[i] - q[2 * i + 1];
+      }
+    }
   }
+}
+
+// Block blk (values 32 blk .. 32 blk + 31, in v; 0 <= blk < 4 kGemmNs) of a row into the row's
+// GemmRecT<NT> record r: one lane per block (split32_fp6_each): the NT terms' codes and scale bytes.
+template <int NT>
+__device__ __forceinline__ void rec_split_block(const float (&v)[32], int blk, uint8_t *r) {
+  using R = GemmRecT<NT>;
+  const int st = blk >> 2, i = blk & 3;
+  split32_fp6_each<NT>(v, [&](int t, const u32x6v &c, uint32_t sb) {
+    *reinterpret_cast<uint4 *>(r + R::dword(st, t, i, 0)) = make_uint4(c[0], c[1], c[2], c[3]);
+    *reinterpret_cast<uint2 *>(r + R::dword(st, t, i, 4)) = make_uint2(c[4], c[5]);
+    r[R::scale(st, t) + i] = (uint8_t)sb;
+  });
 }
 
 // tile_mfma_f8 over steps [s0, s0 + NS) of a tile whose chunks for those steps are in raw[] (zeros

@@ -29,8 +29,8 @@
 // among the loads the compiler would wait for every load, and the ring would drain at each
 // round's end.
 //
-// COLS = 8 (four terms, launch_gemm_fine): chunks of up to 8 entries, MFMA column j = entry j % 8 of
-// term 2 m + j / 8, m = 0, 1; the two halves' sums are added once, in the epilogue.
+// COLS = 8 (six terms, launch_gemm_fine): chunks of up to 8 entries, MFMA column j = entry j % 8 of
+// term 2 m + j / 8, m = 0, 1, 2; the two halves' sums are added once, in the epilogue.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int r = 0; r < RT; r++) {
               const float4 b4 = bias[r];
-              // (four terms: h is exact to 2^-18, so its last bits count)
+              // (six terms: h is exact to 2^-28, so its last bits count)
               const float2 h2 = NT > kGemmTerms ? make_float2(swiglu(acc[r][0] + b4.x, acc[r][1] + b4.y, a.limit),
                                                               swiglu(acc[r][2] + b4.z, acc[r][3] + b4.w, a.limit))
                                                 : make_float2(swiglu_fast(acc[r][0] + b4.x, acc[r][1] + b4.y, a.limit),
@@ -514,23 +514,13 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
                 v[4 * k4 + 2] = x.z;
                 v[4 * k4 + 3] = x.w;
               }
-              float m = 0.0f;
-              bool bad = false;
-#pragma unroll
-              for (int q = 0; q < 32; q++) {
-                m = fmaxf(m, fabsf(v[q]));
-                bad = bad || !isfinite(v[q]);
-              }
-              uint32_t dq[NT][6], sbw;
-              split32_fp6<NT>(v, m, bad, dq, sbw);
               const int hb = cur.grp, st_ = hb >> 2, i = hb & 3;
               uint8_t *hr = reinterpret_cast<uint8_t *>(a.out) + (size_t)(cur.beg + lane) * G::kBytes;
-#pragma unroll
-              for (int tt = 0; tt < NT; tt++) {
-                str_st16(hr + G::dword(st_, tt, i, 0), make_uint4(dq[tt][0], dq[tt][1], dq[tt][2], dq[tt][3]));
-                str_st8(hr + G::dword(st_, tt, i, 4), make_uint2(dq[tt][4], dq[tt][5]));
-                str_st1(hr + G::scale(st_, tt) + i, (sbw >> (8 * tt)) & 0xFFu);
-              }
+              split32_fp6_each<NT>(v, [&](int tt, const u32x6v &c, uint32_t sb) {
+                str_st16(hr + G::dword(st_, tt, i, 0), make_uint4(c[0], c[1], c[2], c[3]));
+                str_st8(hr + G::dword(st_, tt, i, 4), make_uint2(c[4], c[5]));
+                str_st1(hr + G::scale(st_, tt) + i, sb);
+              });
             }
           } else {
             if (j < cur.cnt) {
@@ -581,11 +571,11 @@ bool gemm_stream_local_ok(const GemmArgs &a) {
   return a.n_entries <= (size_t)kLocalGroupMax && a.terms == kGemmTerms && gemm_stream_fits(a, 4, stream_cus());
 }
 
-// Entries per chunk of the four-term form: two of the four terms of eight entries fill the 16 MFMA
-// columns, so a weight chunk feeds two MFMAs and the loader moves half the records of a 16-entry
-// chunk. Measured (20B / 120B layer, us): 7 tokens 68.7 against 73.5 with 16 entries and 68.0 with
-// 4; 31 tokens 96.1 against 104.3 and 113.4 (experts of more than 4 entries stream twice); 120B at
-// 127 tokens 336 against 356 and 421.
+// Entries per chunk of the six-term form: two of the terms of eight entries fill the 16 MFMA columns,
+// so a weight chunk feeds an MFMA per two terms and the loader moves half the records of a 16-entry
+// chunk. Measured with four terms (20B / 120B layer, us): 7 tokens 68.7 against 73.5 with 16 entries
+// and 68.0 with 4; 31 tokens 96.1 against 104.3 and 113.4 (experts of more than 4 entries stream
+// twice); 120B at 127 tokens 336 against 356 and 421.
 constexpr int kFineCols = 8;
 
 bool gemm_fine_fits(const GemmArgs &gu, const PackDims &dn) {
@@ -610,13 +600,16 @@ static int stream_cus() {
   return c;
 }
 
+template <int MODE, int RT, int NSR, int PA, int PB, int NT, int COLS = kStrCols>
+static hipError_t launch_stream(const GemmArgs &a, hipStream_t s, int n_wg) {
+  hipLaunchKernelGGL((k_gemm_stream<MODE, RT, NSR, PA, PB, NT, COLS>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
+  return hipGetLastError();
+}
+
 template <int MODE, int RT, int PA, int PB, int NT, int COLS = kStrCols>
 static hipError_t launch_stream_rt(const GemmArgs &a, hipStream_t s, int n_wg) {
-  if (a.d.ns == 23)
-    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 23, PA, PB, NT, COLS>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_gemm_stream<MODE, RT, 24, PA, PB, NT, COLS>), dim3((unsigned)n_wg), dim3(64 * kStrWaves), 0, s, a);
-  return hipGetLastError();
+  return a.d.ns == 23 ? launch_stream<MODE, RT, 23, PA, PB, NT, COLS>(a, s, n_wg)
+                      : launch_stream<MODE, RT, 24, PA, PB, NT, COLS>(a, s, n_wg);
 }
 
 // The streamed kernel for this launch, or hipErrorNotSupported when it does not fit (the caller
@@ -639,18 +632,20 @@ hipError_t launch_gemm_stream(GemvMode mode, const GemmArgs &a, hipStream_t s, b
   return one ? launch_stream_rt<GEMV_DOWN, 2, 8, 4, 1>(a, s, n_wg) : launch_stream_rt<GEMV_DOWN, 2, 8, 4, kGemmTerms>(a, s, n_wg);
 }
 
-// The four-term form (experts averaging fewer than 4 entries). The weight stream bounds it: at 120B
-// x 48 tokens gate_up reads 0.88 GB in 151 us (5.9 TB/s). A register rings of 4 (gate_up) and 8
-// (down) steps, as the three-term form's 3 and 8. Against the per-tile GEMV on bf16 hi + lo
-// operands, whose weight decode bounds it (us per layer): 20B at 2 tokens 49.8 -> 40.8, 8 tokens
-// 123.7 -> 70.4, 31 tokens 193.4 -> 96.1; 120B at 16 tokens 226.5 -> 144.0, 48 tokens 489 -> 251,
-// 127 tokens 638 -> 336.
+// The six-term form (experts averaging fewer than 4 entries). The weight stream bounds it. A register
+// rings of 4 (gate_up) and 8 (down) steps, as the three-term form's 3 and 8. Against the per-tile GEMV
+// on bf16 hi + lo operands, whose weight decode bounds it (2880 x 2880, top-4, us per layer): 32
+// experts at 2 tokens 48.8 -> 44.5, 8 tokens 136.9 -> 85.8, 31 tokens 186.0 -> 97.4; 128 experts at
+// 16 tokens 209.8 -> 141.9, 48 tokens 462.7 -> 238.7, 127 tokens 616.9 -> 337.1. With four terms, which
+// lose values beside an outlier (kFineTerms), it is about 4 % faster.
 hipError_t launch_gemm_fine(GemvMode mode, const GemmArgs &a, hipStream_t s) {
   const int n_wg = stream_cus();
   if (!a.n_entries) return hipSuccess;
   if (a.terms != kFineTerms || !gemm_stream_fits(a, mode == GEMV_GATE_UP ? 4 : 2, n_wg, kFineCols)) return hipErrorInvalidValue;
-  return mode == GEMV_GATE_UP ? launch_stream_rt<GEMV_GATE_UP, 4, 4, 4, kFineTerms, kFineCols>(a, s, n_wg)
-                              : launch_stream_rt<GEMV_DOWN, 2, 8, 4, kFineTerms, kFineCols>(a, s, n_wg);
+  if (mode == GEMV_DOWN) return launch_stream_rt<GEMV_DOWN, 2, 8, 4, kFineTerms, kFineCols>(a, s, n_wg);
+  // (one step less at run-time step counts, whose kernel otherwise spills)
+  return a.d.ns == 23 ? launch_stream<GEMV_GATE_UP, 4, 23, 4, 4, kFineTerms, kFineCols>(a, s, n_wg)
+                      : launch_stream<GEMV_GATE_UP, 4, 24, 3, 4, kFineTerms, kFineCols>(a, s, n_wg);
 }
 
 }  // namespace moe

@@ -84,18 +84,22 @@ constexpr int kTerms = 4;
 // then dwords 4-5 of blocks 0..3 (8 bytes each, at 64 + 8 b); then [term t][4 scale bytes, byte
 // i = E8M0 of block 4s+i] (4 NT bytes) and pad bytes to 16. A step is kChunks 16-byte chunks:
 // chunk 6t + b = the first 16 bytes of block b, chunk 6t + 4 + (b >> 1) = the last 8 bytes of
-// blocks b and b ^ 1, chunk 6 NT = the scales (the grouped GEMM stages them chunk by chunk).
-// Blocks past the row are zero. NT = kGemmTerms: the exact split (the default); NT = kFineTerms: one
-// term more (2^-18 of a block's maximum), for batches whose experts average fewer than 4 entries;
-// NT = 1: the quantized-activation mode (one MXFP6 term per value).
+// blocks b and b ^ 1, from chunk 6 NT the scales (the grouped GEMM stages them chunk by chunk).
+// Blocks past the row are zero. NT = kGemmTerms: the exact split (the default); NT = kFineTerms:
+// 2^-28 of a block's maximum, for batches whose experts average fewer than 4 entries; NT = 1: the
+// quantized-activation mode (one MXFP6 term per value).
 constexpr int kGemmNs = 24;
 constexpr int kGemmTerms = 3;
-constexpr int kFineTerms = 4;
+// Six terms keep every value down to 2^-11 of its block's maximum to the 2^-17 of itself that bf16
+// hi + lo operands keep; four (2^-18 of the maximum) served ordinary values better than those but
+// lost values beside an outlier (2880 x 2880, 7 tokens, error of a layer with one channel at 1000
+// times the rest: bf16 2.3e-6, four terms 5.7e-6; at 1e5 times 3.5e-7 and 4.6e-4).
+constexpr int kFineTerms = 6;
 template <int NT>
 struct GemmRecT {
   static constexpr int kNT = NT;
   static constexpr int kTermBytes = 96;
-  static constexpr int kStep = NT * kTermBytes + 16;
+  static constexpr int kStep = NT * kTermBytes + (4 * NT + 15) / 16 * 16;
   static constexpr int kChunks = kStep / 16;
   static constexpr int kBytes = kGemmNs * kStep;
   // byte offset of dword d (0..5) of the B operand of block b (0..3) of step s, term t
@@ -103,7 +107,7 @@ struct GemmRecT {
     return s * kStep + t * kTermBytes + (d < 4 ? 16 * b + 4 * d : 64 + 8 * b + 4 * (d - 4));
   }
   MOE_HD static constexpr int scale(int s, int t) { return s * kStep + NT * kTermBytes + 4 * t; }
-  static_assert(NT >= 1 && NT <= 4 && kStep % 16 == 0 && kChunks == 6 * NT + 1, "record chunks");
+  static_assert(NT >= 1 && NT <= 8 && kStep % 16 == 0 && kChunks == 6 * NT + (NT + 3) / 4, "record chunks");
 };
 using GemmRec = GemmRecT<kGemmTerms>;
 
@@ -143,7 +147,7 @@ hipError_t launch_gemm_fp8(GemvMode mode, const GemmArgs &a, hipStream_t s);
 // when the launch does not fit it.
 hipError_t launch_gemm_stream(GemvMode mode, const GemmArgs &a, hipStream_t s, bool alt);
 // The streamed form with kFineTerms terms, for batches whose experts average fewer than 4 entries
-// (activations to 2^-18 of a block's maximum); gemm_fine_fits: whether both GEMMs of the layer
+// (activations to 2^-28 of a block's maximum); gemm_fine_fits: whether both GEMMs of the layer
 // (gu: the gate_up arguments; dn: the down matrix) and its local grouping take this batch.
 bool gemm_fine_fits(const GemmArgs &gu, const PackDims &dn);
 hipError_t launch_gemm_fine(GemvMode mode, const GemmArgs &a, hipStream_t s);

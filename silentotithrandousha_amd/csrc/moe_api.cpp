@@ -237,11 +237,11 @@ size_t router_bytes(size_t H, size_t E) { return E * 64 * router_kip(H) * 2; }
 // Lays out the per-call workspace of T tokens, top-k k and E experts at `b` (nullptr: sizes
 // only) and returns its bytes. host_io adds the staging rows of host-pointer calls (x, y) and
 // the normalised row of the single token's unfused block forward (xn).
-// what: with WORK_FINE only the operands of the four-term small-batch GEMM, with WORK_COARSE those
+// what: with WORK_FINE only the operands of the six-term small-batch GEMM, with WORK_COARSE those
 // of the other paths.
 size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size_t I, bool host_io, WorkFor what) {
   const size_t N = T * k;
-  // the four-term GEMM takes batches of fewer than 4 E entries
+  // the six-term GEMM takes batches of fewer than 4 E entries
   const size_t NF = what == WORK_COARSE ? 0 : std::min(N, 4 * E), TF = what == WORK_COARSE ? 0 : std::min(T, 4 * E);
   const size_t NC = what == WORK_FINE ? 0 : N, TC = what == WORK_FINE ? 0 : T;
   size_t off = 0;
@@ -478,7 +478,7 @@ GemmArgs gemm_args(const moe_ctx *c, const Layer &Ly, size_t T, size_t k) {
   return ga;
 }
 
-// Whether a batch runs the four-term streamed GEMM: experts averaging fewer than 4 entries, where
+// Whether a batch runs the six-term streamed GEMM: experts averaging fewer than 4 entries, where
 // the weights are read about once per entry and the three-term split of the larger batches would
 // be less exact than the bf16 hi + lo operands of the GEMV path that it replaces.
 bool takes_fine(const moe_ctx *c, const Layer &Ly, size_t T, size_t k, const float *x) {
@@ -1094,7 +1094,7 @@ int moe_layer_forward_device_noalloc(moe_ctx *c, size_t layer, const float *x, s
   if (!c->scratch) return fail(MOE_ERR_STATE, "no scratch array address for device %d", c->dev);
   const size_t E = c->layers[layer].n_experts;
   Work w{};
-  // a batch of the four-term GEMM whose operands the array does not hold takes the other path
+  // a batch of the six-term GEMM whose operands the array does not hold takes the other path
   WorkFor what = takes_fine(c, c->layers[layer], T, k, x) ? WORK_FINE : WORK_COARSE;
   if (what == WORK_FINE && carve_work(w, nullptr, T, k, E, c->H, c->I, false, what) > noalloc_scratch_bytes()) what = WORK_COARSE;
   const size_t need = carve_work(w, nullptr, T, k, E, c->H, c->I, false, what);

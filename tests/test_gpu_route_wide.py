@@ -42,6 +42,6 @@ def test_wide_router_bit_exact(orc, H, E, k, T):
         big = d.layer_forward(0, x, k)
         parts = np.concatenate([d.layer_forward(0, x[i:i + 64], k) for i in range(0, T, 64)])
         assert k == 1 or n_dropped > 0
-        assert_rel_l2(big, parts, "adaptive", 3e-4)  # the batches may take GEMMs of 3 or 4 terms: 2^-13 of a block
+        assert_rel_l2(big, parts, "adaptive", 3e-4)  # the batches may take GEMMs of 3 or 6 terms: 2^-13 of a block
     finally:
         d.close()
