@@ -78,11 +78,11 @@ int moe_set_adaptive_topk(moe_ctx *ctx, int enabled, size_t min_k, float top1_mi
  * moe_layer_forward return MOE_ERR_HIP (which clears the condition).
  * MOE_OPT_BATCH_GEMM: batches (n_tokens > 1) run through the grouped GEMM on the block-scaled
  * MFMA when 1 (default): activations as 3 fp6 terms, exact to 2^-13 of a block's maximum, once
- * experts average at least 4 entries, and as 6 terms, exact to 2^-28, below that (the streamed
- * form of code 12 with 8-entry chunks; MOE_OPT_GEMM_SHAPE and MOE_OPT_ACT_QUANT do not apply to
- * it). 2: always the 3-term form. 0, and batches that the grouped GEMM does not take (K above
- * 3072, x not 16-byte aligned, fewer than 96 rows): the per-tile GEMV kernels (bf16 hi+lo
- * activations). Results agree to the matmul tolerance; routing is identical.
+ * experts average at least 4 entries, and as 6 terms, exact to 2^-28, below that where the weights
+ * that the tokens choose are large enough (tens of MB; the streamed form of code 12 with 8-entry
+ * chunks; MOE_OPT_GEMM_SHAPE and MOE_OPT_ACT_QUANT do not apply to it). 2: always the 3-term form.
+ * 0, and the other batches (fewer weights, K above 3072, x not 16-byte aligned): the per-tile GEMV
+ * kernels (bf16 hi+lo activations). Results agree to the matmul tolerance; routing is identical.
  * MOE_OPT_GEMM_SHAPE: block shape of the grouped GEMM: 0 (default) by the mean entries per
  * expert (14 to 44, 60 to 72, and for the down GEMM 14 to 72: the wide streamed form of code 14;
  * otherwise 48+: 512 rows x 64 entries in 8 wavefronts, at K of 2817-3072 with the pipelined step

@@ -478,13 +478,33 @@ GemmArgs gemm_args(const moe_ctx *c, const Layer &Ly, size_t T, size_t k) {
   return ga;
 }
 
-// Whether a batch runs the six-term streamed GEMM: experts averaging fewer than 4 entries, where
-// the weights are read about once per entry and the three-term split of the larger batches would
-// be less exact than the bf16 hi + lo operands of the GEMV path that it replaces.
+// Whether the six-term streamed GEMM is ahead of the GEMV kernels for T tokens at top-k of E experts.
+// A launch of it costs about 8 us more and, at any K, 24 loop positions per round of 4 units; it gains
+// from the weights, which the GEMV decodes once more for every 8 (16, 32) entries. So: by an expert's
+// bytes and those of all experts that T tokens are expected to choose. Measured over 17 shapes of 512
+// to 3072 values, 8 to 256 experts, top-1 to 4, 2 to 511 tokens (2618 points; us a layer, GEMV
+// against this): 512 x 512 always behind (127 tokens, 128 experts: 45 / 56); 1024 x 1024 and 128
+// experts at 24 tokens 68 / 71, at 127 114 / 100; 3072 x 512 and 8 experts at 31 tokens 42 / 35; 2304 x
+// 2304 and 32 experts at 2 tokens 35 / 41, at 9 76 / 64; 2880 x 2880 and 32 experts at 2 tokens top-1
+// 30 / 37, top-4 49 / 45. u: units a workgroup, in rounds; just over one round leaves most of the
+// second one empty (1792 x 1792, 32 experts, 9 tokens: 50 / 58). Where the rule takes this form it is
+// 1.30 times as fast in the mean, and behind by more than 2 % at 18 of 1195 points (at most 8 %).
+bool fine_ahead(const ExpertLayout &L, size_t E, size_t T, size_t k) {
+  const double e = 1e-6 * (double)(pack_weight_bytes(L.gu) + pack_weight_bytes(L.dn)) * 17 / 16;  // MB, with scales
+  const double active = (double)E * (1.0 - std::pow(1.0 - (double)k / (double)E, (double)T)), all = active * e;
+  if (T > 16) return all >= (e >= 2.4 ? 18.0 : e >= 1.6 ? 120.0 : HUGE_VAL);  // the GEMV computes 32 columns or more
+  if (e >= 8.0) return all >= (T <= 3 ? 80.0 : 62.0);
+  const double u = active * (L.gu.tiles / 4) / 1024;
+  return e >= 4.9 && all >= 85.0 && !(u > 1.0 && u < 1.75);
+}
+
+// Whether a batch runs the six-term streamed GEMM: experts averaging fewer than 4 entries (where the
+// three-term split of the larger batches would be less exact than the bf16 hi + lo operands of the
+// GEMV path that it replaces), and enough weights for it to be ahead of that path.
 bool takes_fine(const moe_ctx *c, const Layer &Ly, size_t T, size_t k, const float *x) {
   return c->batch_gemm == 1 && T > 1 && T * k < 4 * Ly.n_experts && c->L.gu.ns <= (uint32_t)kGemmNs &&
          c->L.dn.ns <= (uint32_t)kGemmNs && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-         gemm_fine_fits(gemm_args(c, Ly, T, k), c->L.dn);
+         fine_ahead(c->L, Ly.n_experts, T, k) && gemm_fine_fits(gemm_args(c, Ly, T, k), c->L.dn);
 }
 
 // norm: the block forward (RMSNorm of x before, x + result after). The one-launch decode fuses
@@ -598,9 +618,10 @@ int forward_device(moe_ctx *c, const Work &w, size_t layer, const float *x, size
   ra.logits = w.logits;
   ra.idx = w.idx;
   ra.wts = w.wts;
-  // the grouped GEMM (16- to 64-entry column tiles) pays off once experts average a few
-  // entries; smaller batches stream each weight tile through the GEMV kernels, which read the
-  // bf16 hi + lo split of x that the router writes
+  // the grouped GEMM (16- to 64-entry column tiles) pays off once experts average a few entries,
+  // its six-term form below that where the weights are large (takes_fine); other batches stream
+  // each weight tile through the GEMV kernels, which read the bf16 hi + lo split of x that the router
+  // writes
   // (unaligned x rows take the GEMV path, unless the router writes normalised ones)
   const float *rows = route_norm ? w.xn : x;
   const bool fine = w.hfine && takes_fine(c, Ly, T, k, rows);

@@ -27,18 +27,19 @@ def _pair(d, x, k):
     return got, ref
 
 
-# H, I, E, k, T, router sigma: one and two K-step quads, K not a multiple of 128, the smallest shape the
-# streamed form takes (3 units per chunk) and one it refuses (64), 23 and 24 steps, 256 experts,
-# top-1, experts of 1 to 8, 9 and 17 entries (a large router spread sends every token to the
-# same experts), the largest average below 4
-CASES = [(96, 96, 8, 2, 5, 0.1), (64, 64, 8, 4, 3, 0.1), (160, 224, 8, 1, 31, 0.1), (512, 512, 64, 4, 50, 0.1),
-         (2880, 2880, 8, 4, 2, 0.1), (3072, 1056, 8, 4, 7, 0.1), (256, 3072, 32, 4, 31, 0.1),
-         (256, 128, 256, 4, 255, 0.1), (256, 256, 32, 4, 8, 40.0), (256, 256, 32, 4, 9, 40.0),
-         (256, 256, 32, 4, 17, 40.0)]
+# H, I, E, k, T, router sigma: the forms the rule (fine_ahead) takes: 23 and 24 steps, K not a multiple of
+# 128 on either side, the smallest experts, 128 and 256 experts, experts of 1 to 8, 9, 17 and 31 entries (a
+# large router spread sends every token to the same experts), the largest average below 4
+FINE = [(2880, 2880, 8, 4, 6, 0.1), (3072, 3072, 8, 4, 3, 0.1), (3072, 1056, 8, 1, 31, 0.1), (544, 3072, 8, 1, 31, 0.1),
+        (3040, 512, 8, 1, 31, 0.1), (2080, 2432, 16, 2, 12, 0.1), (1024, 1024, 128, 4, 48, 0.1), (352, 3072, 256, 1, 200, 0.1),
+        (2304, 2304, 16, 2, 8, 40.0), (2304, 2304, 16, 2, 9, 40.0), (2304, 2304, 16, 2, 17, 40.0), (2304, 2304, 16, 2, 31, 40.0)]
+# and forms it leaves to the GEMV: small experts at any count of tokens, few weights in all, K past 3072
+GEMV = [(96, 96, 8, 2, 5, 0.1), (64, 64, 8, 4, 3, 0.1), (160, 224, 8, 1, 31, 0.1), (512, 512, 64, 4, 50, 0.1),
+        (256, 256, 32, 4, 31, 0.1), (256, 128, 256, 4, 255, 0.1), (2880, 2880, 8, 1, 2, 0.1), (3104, 1056, 8, 1, 31, 0.1)]
 
 
-@pytest.mark.parametrize("H,I,E,k,T,sigma", CASES)
-def test_small_batch_matches_oracle_and_gemv(orc, H, I, E, k, T, sigma):
+@pytest.mark.parametrize("H,I,E,k,T,sigma,fine", [c + (True,) for c in FINE] + [c + (False,) for c in GEMV])
+def test_small_batch_matches_oracle_and_gemv(orc, H, I, E, k, T, sigma, fine):
     assert T * k < 4 * E
     L = syn.make_layer(H, I, E, seed=600 + T + H, scale_lo=117, scale_hi=121, router_sigma=sigma)
     d = GpuMoeDispatcher(H, I, 7.0)
@@ -48,13 +49,14 @@ def test_small_batch_matches_oracle_and_gemv(orc, H, I, E, k, T, sigma):
         if sigma > 1:
             x = x[:1] + 1e-3 * x  # tokens alike: the same experts for all of them
         got, ref = _pair(d, x, k)
+        assert np.array_equal(got, ref) != fine  # which of the two ran: their last bits differ
         want, _, idx, _ = orc.moe_layer(x, L, k)
         gidx, _ = d.router_topk(0, x, k)
         assert np.array_equal(gidx, idx)
         if sigma > 1:
             assert np.bincount(idx[idx >= 0].ravel()).max() == T
-        e_new, e_gemv = assert_rel_l2(got, want, "six terms", 2e-5), assert_rel_l2(ref, want, "GEMV", 2e-5)
-        print(f"oracle: six terms {e_new:.2e}, GEMV {e_gemv:.2e}; apart {rel_l2(got, ref):.2e}")
+        e_new, e_gemv = assert_rel_l2(got, want, "default", 2e-5), assert_rel_l2(ref, want, "GEMV", 2e-5)
+        print(f"oracle: default {e_new:.2e}, GEMV {e_gemv:.2e}; apart {rel_l2(got, ref):.2e}")
         assert rel_l2(got, ref) < GEMV_TOL
         d.set_local_group(0)  # grouped by the router instead of the GEMM's workgroups
         assert np.array_equal(d.layer_forward(0, x, k), got)
@@ -65,9 +67,9 @@ def test_small_batch_matches_oracle_and_gemv(orc, H, I, E, k, T, sigma):
 def test_small_batch_outliers_and_extremes(orc):
     """Activations that a block scale serves worst: one value of a block a thousand times the rest,
     magnitudes from 2^-100 to 2^60, zero rows, and a non-finite value (NaN in its token alone)."""
-    H, I, E, k = 512, 256, 16, 2
+    H, I, E, k, T = 3072, 512, 8, 1, 31
     L = syn.make_layer(H, I, E, seed=640, scale_lo=117, scale_hi=121, router_sigma=0.1)
-    x = syn.hidden(9, H, seed=641)
+    x = syn.hidden(T, H, seed=641)
     x[0, ::32] *= 1000.0
     x[1] *= np.float32(2.0**-100)
     x[2, :64] *= np.float32(2.0**60)
@@ -76,14 +78,15 @@ def test_small_batch_outliers_and_extremes(orc):
     try:
         d.preload_layer(0, L)
         got, ref = _pair(d, x, k)
+        assert not np.array_equal(got, ref)
         want = orc.moe_layer(x, L, k)[0]
-        for t in range(9):
+        for t in range(T):
             assert_rel_l2(got[t], want[t], f"token {t}", 2e-5)
             assert rel_l2(got[t], ref[t]) < GEMV_TOL
         x[4, 7] = np.nan
         bad = d.layer_forward(0, x, k)
         assert not np.isfinite(bad[4]).any()
-        keep = [t for t in range(9) if t != 4]
+        keep = [t for t in range(T) if t != 4]
         assert np.array_equal(bad[keep], got[keep])
     finally:
         d.close()
@@ -94,16 +97,17 @@ def test_small_batch_values_beside_an_outlier(orc, gain):
     """Every block of x holds one value `gain` times the rest, which no weight reads: the outputs are the
     small values' alone. Within the bound of the bf16 hi + lo operands (2^-17 of each value); terms cut
     at 2^-18 of the block's maximum were 4e-5 and 3e-4 off."""
-    H, I, E, k = 512, 256, 16, 2
+    H, I, E, k = 3072, 512, 8, 1
     L = syn.make_layer(H, I, E, seed=645, scale_lo=117, scale_hi=121, router_sigma=0.1)
     L["gu_blocks"][..., 0] &= 0xF0  # value 0 of each block of 32
-    x = syn.hidden(9, H, seed=646)
+    x = syn.hidden(31, H, seed=646)
     x[:, ::32] *= gain
     d = GpuMoeDispatcher(H, I, 7.0)
     try:
         d.preload_layer(0, L)
         got, ref = _pair(d, x, k)
         want = orc.moe_layer(x, L, k)[0]
+        assert not np.array_equal(got, ref)
         assert_rel_l2(ref, want, "GEMV", 8e-6)
         assert_rel_l2(got, want, "six terms", 8e-6)
     finally:
@@ -113,7 +117,7 @@ def test_small_batch_values_beside_an_outlier(orc, gain):
 def test_small_batch_adaptive_unaligned_and_replayed(orc):
     """Adaptive top-k's dropped slots; an x that is not 16-byte aligned (the GEMV path); a graph
     captured after one eager call, replayed between eager calls of other sizes."""
-    H, I, E = 256, 128, 32
+    H, I, E = 1024, 1536, 32
     L = syn.make_layer(H, I, E, seed=650, scale_lo=117, scale_hi=121, router_sigma=0.2)
     d = GpuMoeDispatcher(H, I, 7.0)
     try:
@@ -123,6 +127,7 @@ def test_small_batch_adaptive_unaligned_and_replayed(orc):
         want, _, idx, _ = orc.moe_layer(x, L, 4, adaptive=orc.Adaptive(1, 1, 0.7, 0.4, 0.85))
         assert (idx < 0).any()
         got, ref = _pair(d, x, 4)
+        assert not np.array_equal(got, ref)
         assert_rel_l2(got, want, "adaptive", 2e-5)
         assert rel_l2(got, ref) < GEMV_TOL
         d.set_adaptive_topk(False)
