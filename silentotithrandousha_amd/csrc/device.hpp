@@ -989,8 +989,8 @@ __device__ __forceinline__ void split32_fp6_each(const float (&x)[32], F &&emit)
   }
 }
 
-// Block blk (values 32 blk .. 32 blk + 31, in v; 0 <= blk < 4 kGemmNs) of a row into the row's
-// GemmRecT<NT> record r: one lane per block (split32_fp6_each): the NT terms' codes and scale bytes.
+// Block blk (values 32 blk .. 32 blk + 31, in v; of a step that the record holds) of a row into the
+// row's GemmRecT<NT> record r: one lane per block (split32_fp6_each): the NT terms' codes and scale bytes.
 template <int NT>
 __device__ __forceinline__ void rec_split_block(const float (&v)[32], int blk, uint8_t *r) {
   using R = GemmRecT<NT>;

@@ -341,11 +341,11 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
         const int c = min(64 * pc + lane, COLS * G::kChunks - 1);
         real[i] = ar == 0 || t.two;
         const int qa = min(t.qf + ar, kStrMaxSeg - 1);
-        off[i] = real[i] ? (uint32_t)s_row[qa][c / G::kChunks] * (uint32_t)G::kBytes + 16u * (c % G::kChunks) : 0u;
+        off[i] = real[i] ? (uint32_t)s_row[qa][c / G::kChunks] * (uint32_t)G::row_bytes(ns) + 16u * (c % G::kChunks) : 0u;
       }
     };
     auto load_b = [&](const uint32_t (&off)[L::kDma], const bool (&real)[L::kDma], int s, int sl) {
-      const uint8_t *bs = a.brec + (size_t)min(s, kGemmNs - 1) * G::kStep;
+      const uint8_t *bs = a.brec + (size_t)min(s, (NT == kFineTerms ? ns : kGemmNs) - 1) * G::kStep;
 #pragma unroll
       for (int i = 0; i < L::kDma; i++)
         str_dma16(off[i], bs, real[i] ? str_lds(&sB[sl][i / kPieces][(i % kPieces) * 1024]) : str_lds(sBd));
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(64 * kStrWaves) __attribute__((amdgpu_waves_per_eu(
                 v[4 * k4 + 3] = x.w;
               }
               const int hb = cur.grp, st_ = hb >> 2, i = hb & 3;
-              uint8_t *hr = reinterpret_cast<uint8_t *>(a.out) + (size_t)(cur.beg + lane) * G::kBytes;
+              uint8_t *hr = reinterpret_cast<uint8_t *>(a.out) + (size_t)(cur.beg + lane) * G::row_bytes((Gu + 3) / 4);
               split32_fp6_each<NT>(v, [&](int tt, const u32x6v &c, uint32_t sb) {
                 str_st16(hr + G::dword(st_, tt, i, 0), make_uint4(c[0], c[1], c[2], c[3]));
                 str_st8(hr + G::dword(st_, tt, i, 4), make_uint2(c[4], c[5]));

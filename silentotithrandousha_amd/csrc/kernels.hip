@@ -227,9 +227,9 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
   // threads u0, u0 + stride, ... (after the router, beside the top-k: off the critical path)
   auto write_records = [&](int u0, int stride) {
     if (!a.xrec) return;
-    constexpr int kRecBlocks = 4 * kGemmNs;
-    for (int u = u0; u < nt * kRecBlocks; u += stride) {
-      const int tb = u / kRecBlocks, blk = u - tb * kRecBlocks, k0 = 32 * blk;
+    const int ns = (H + 127) / 128, nrec = NT == kFineTerms ? 4 * ns : 4 * kGemmNs;
+    for (int u = u0; u < nt * nrec; u += stride) {
+      const int tb = u / nrec, blk = u - tb * nrec, k0 = 32 * blk;
       const float *xt = s_x + tb * Hp;
       float xv[32];
 #pragma unroll
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
         xv[4 * q + 2] = k0 + 4 * q + 2 < H ? x4.z : 0.0f;
         xv[4 * q + 3] = k0 + 4 * q + 3 < H ? x4.w : 0.0f;
       }
-      rec_split_block<NT>(xv, blk, a.xrec + (size_t)(t0 + tb) * GemmRecT<NT>::kBytes);
+      rec_split_block<NT>(xv, blk, a.xrec + (size_t)(t0 + tb) * GemmRecT<NT>::row_bytes(ns));
     }
   };
   if constexpr (KI > 0) {

@@ -102,6 +102,9 @@ struct GemmRecT {
   static constexpr int kStep = NT * kTermBytes + (4 * NT + 15) / 16 * 16;
   static constexpr int kChunks = kStep / 16;
   static constexpr int kBytes = kGemmNs * kStep;
+  // Bytes of the record of a row of ns K-steps: kFineTerms records hold these steps only (as many rows
+  // then fit a workspace as of the operands of the other paths), the others all kGemmNs.
+  MOE_HD static constexpr int row_bytes(int ns) { return NT == kFineTerms ? ns * kStep : kBytes; }
   // byte offset of dword d (0..5) of the B operand of block b (0..3) of step s, term t
   MOE_HD static constexpr int dword(int s, int t, int b, int d) {
     return s * kStep + t * kTermBytes + (d < 4 ? 16 * b + 4 * d : 64 + 8 * b + 4 * (d - 4));

@@ -267,11 +267,11 @@ size_t carve_work(Work &w, char *b, size_t T, size_t k, size_t E, size_t H, size
   w.blk_count = (int32_t *)take(T * E * 4);  // router blocks <= T
   w.rank = (int32_t *)take(N * 4);
   w.xrec = (uint8_t *)take(TC * GemmRec::kBytes);
-  w.xfine = (uint8_t *)take(TF * GemmRecT<kFineTerms>::kBytes);
+  w.xfine = (uint8_t *)take(TF * GemmRecT<kFineTerms>::row_bytes((int)((H + 127) / 128)));
   // the h records last, one after the other: cleared together
   w.hrec_bytes = NC * GemmRec::kBytes;
   w.hrec = (uint8_t *)take(w.hrec_bytes);
-  w.hfine_bytes = NF * GemmRecT<kFineTerms>::kBytes;
+  w.hfine_bytes = NF * GemmRecT<kFineTerms>::row_bytes((int)((I + 127) / 128));
   w.hfine = (uint8_t *)take(w.hfine_bytes);
   return off;
 }
@@ -488,7 +488,7 @@ GemmArgs gemm_args(const moe_ctx *c, const Layer &Ly, size_t T, size_t k) {
 // 2304 and 32 experts at 2 tokens 35 / 41, at 9 76 / 64; 2880 x 2880 and 32 experts at 2 tokens top-1
 // 30 / 37, top-4 49 / 45. u: units a workgroup, in rounds; just over one round leaves most of the
 // second one empty (1792 x 1792, 32 experts, 9 tokens: 50 / 58). Where the rule takes this form it is
-// 1.30 times as fast in the mean, and behind by more than 2 % at 18 of 1195 points (at most 8 %).
+// 1.31 times as fast in the mean, and behind by more than 2 % at 16 of 1188 points (at most 8 %).
 bool fine_ahead(const ExpertLayout &L, size_t E, size_t T, size_t k) {
   const double e = 1e-6 * (double)(pack_weight_bytes(L.gu) + pack_weight_bytes(L.dn)) * 17 / 16;  // MB, with scales
   const double active = (double)E * (1.0 - std::pow(1.0 - (double)k / (double)E, (double)T)), all = active * e;
@@ -1115,9 +1115,9 @@ int moe_layer_forward_device_noalloc(moe_ctx *c, size_t layer, const float *x, s
   if (!c->scratch) return fail(MOE_ERR_STATE, "no scratch array address for device %d", c->dev);
   const size_t E = c->layers[layer].n_experts;
   Work w{};
-  // a batch of the six-term GEMM whose operands the array does not hold takes the other path
-  WorkFor what = takes_fine(c, c->layers[layer], T, k, x) ? WORK_FINE : WORK_COARSE;
-  if (what == WORK_FINE && carve_work(w, nullptr, T, k, E, c->H, c->I, false, what) > noalloc_scratch_bytes()) what = WORK_COARSE;
+  // (the six-term GEMM's operands are the smaller ones: 608 bytes of records against 304 + 512 of
+  // records and bf16 rows per 128 values)
+  const WorkFor what = takes_fine(c, c->layers[layer], T, k, x) ? WORK_FINE : WORK_COARSE;
   const size_t need = carve_work(w, nullptr, T, k, E, c->H, c->I, false, what);
   if (need > noalloc_scratch_bytes())
     return fail(MOE_ERR_INVALID,

@@ -44,6 +44,34 @@ def test_noalloc_matches_device_forward(orc):
     d.close()
 
 
+def test_noalloc_small_batches_of_many_experts():
+    """Batches of the six-term GEMM up to what the scratch array held before that path existed (bf16 rows
+    and 3-term records of 560 tokens): the same bits as the allocating forward, also after a call that
+    laid the array out for the GEMV path (x 4 bytes off) and with an I that ends inside a K-step."""
+    H, I, E = 1024, 992, 256
+    L = syn.make_layer(H, I, E, seed=530, scale_lo=117, scale_hi=121, router_sigma=0.1)
+    d = GpuMoeDispatcher(H, I, 7.0)
+    try:
+        d.preload_layer(0, L)
+        na, ref = lib().moe_layer_forward_device_noalloc, lib().moe_layer_forward_device
+        for T, off in ((560, 0), (100, 4), (300, 0), (100, 0), (101, 4)):
+            x = syn.hidden(T, H, seed=531 + T)
+            xd = DeviceBuffer.from_array(np.concatenate([np.zeros(off // 4, np.float32), x.ravel()]))
+            outs = []
+            for fn in (na, ref):
+                yd = DeviceBuffer(x.nbytes)
+                check(fn(d.ctx, 0, ctypes.c_void_p(xd.ptr + off), T, 1, ctypes.c_void_p(yd.ptr), None))
+                d.synchronize()
+                outs.append(yd.download(np.float32, x.shape))
+            assert_bit_exact(outs[0], outs[1], f"T={T} offset {off}")
+            d.set_batch_gemm(0)
+            gemv = d.layer_forward(0, x, 1)
+            d.set_batch_gemm(1)
+            assert np.array_equal(outs[0], gemv) == (off != 0)  # which path ran
+    finally:
+        d.close()
+
+
 def test_noalloc_two_contexts_one_device():
     """Two contexts on one GPU use the same scratch array one after the other: each call's result
     equals its own context's allocating forward."""
