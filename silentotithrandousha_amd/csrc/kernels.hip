@@ -27,6 +27,7 @@ namespace moe {
 
 constexpr int kRouteThreads = 1024;
 constexpr int kRouteTokens = 8;  // tokens per block for large batches: the router weights load once per block
+constexpr size_t kRouteLds = 144 * 1024;  // most dynamic LDS of such a block (its static arrays take 11 KB)
 
 // Groups the T*k (token, slot) entries by expert, in one block of 1024 threads. Active
 // experts are listed in ascending id; entries of one expert are ordered by t*k + slot.
@@ -472,9 +473,9 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(RouteArgs a) {
 
 template <int KI, int TB, int NT, bool NORM>
 static hipError_t launch_route_norm(const RouteArgs &a, size_t hp, hipStream_t s) {
-  if (TB * hp > 65536) {  // more than the default 64 KB of dynamic LDS
+  if (TB > 1) {  // more than the default 64 KB with the static arrays; KI = 0 serves rows of several lengths
     static DynLdsOnce once;
-    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, TB, NT, NORM>), TB * hp);
+    const hipError_t e = ensure_dyn_lds(once, reinterpret_cast<const void *>(&k_route<KI, TB, NT, NORM>), kRouteLds);
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL((k_route<KI, TB, NT, NORM>), dim3((unsigned)((a.T + TB - 1) / TB)), dim3(kRouteThreads), TB * hp, s, a);
@@ -490,7 +491,7 @@ template <int KI>
 static hipError_t launch_route_ki(const RouteArgs &a, int nq, hipStream_t s) {
   const size_t hp = (size_t)nq * 8 * 64 * sizeof(float);
   const int nt = a.xrec ? a.rec_terms : kGemmTerms;
-  if (a.T >= 2048 && kRouteTokens * hp <= 144 * 1024) {
+  if (a.T >= 2048 && kRouteTokens * hp <= kRouteLds) {
     if (nt == 1) return launch_route_tb<KI, kRouteTokens, 1>(a, hp, s);
     if (nt == kGemmTerms) return launch_route_tb<KI, kRouteTokens, kGemmTerms>(a, hp, s);
   }

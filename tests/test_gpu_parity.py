@@ -795,8 +795,9 @@ def test_prefill_2048_tokens_120b(orc):
 # ---------------------------------------------------------------- quantized activations (opt-in)
 
 def test_prefill_partial_router_block_20b(orc, disp20, layer20):
-    """2053 tokens, a multiple of 8 plus 5: the last 8-token router block holds 5 tokens (its
-    idle top-k wavefronts and the wavefronts that write the GEMM records see a partial block).
+    """2053 tokens, a multiple of 16 plus 5: the last workgroup of the wide router holds 5 tokens (its
+    idle top-k wavefronts and the wavefronts that write the GEMM records see a partial block; the
+    8-token blocks of the other router: test_gpu_route_blocks.py).
     Top-k indices of every token exact against the oracle's router; tokens of the first, the
     last full and the partial block within the tolerance of the oracle, on the exact path and on
     the quantized one (against the MXFP6 oracle)."""

@@ -32,7 +32,8 @@ def test_wide_router_bit_exact(orc, H, E, k, T):
         want, _, _, _ = orc.moe_layer(x, L, k)
         assert_rel_l2(d.layer_forward(0, x, k), want, "layer")
         # a prefix below the kernel's range takes the other router: the same tokens, the same bits
-        assert np.array_equal(d.router_topk(0, x, k)[0][:40], d.router_topk(0, x[:40], k)[0])
+        for a, b in zip(d.router_topk(0, x, k, want_logits=True, n_experts=E), d.router_topk(0, x[:40], k, want_logits=True, n_experts=E)):
+            assert np.array_equal(a[:40], b)
         gamma = np.linspace(0.5, 1.5, H).astype(np.float32)
         d.preload_norm(0, gamma, 1e-5)
         n = orc.rms_norm(x, gamma, 1e-5)
@@ -43,5 +44,33 @@ def test_wide_router_bit_exact(orc, H, E, k, T):
         parts = np.concatenate([d.layer_forward(0, x[i:i + 64], k) for i in range(0, T, 64)])
         assert k == 1 or n_dropped > 0
         assert_rel_l2(big, parts, "adaptive", 3e-4)  # the batches may take GEMMs of 3 or 6 terms: 2^-13 of a block
+    finally:
+        d.close()
+
+
+@pytest.mark.parametrize("T", [767, 768, 769])
+def test_switch_to_the_wide_router(orc, T):
+    """The two routers on either side of the switch give the same bits; which one ran shows in the launches:
+    32 experts' grouping does not fit k_route's LDS at this hidden size, so it needs k_bucket (kernel 1),
+    which the wide router's own grouping does without."""
+    H, E, k = 256, 32, 2
+    L = syn.make_layer(H, 96, E, seed=830, scale_lo=117, scale_hi=121, router_sigma=0.1)
+    d = GpuMoeDispatcher(H, 96, 7.0)
+    try:
+        d.preload_layer(0, L)
+        x = syn.hidden(T, H, seed=831)
+        d.set_timing(True)
+        d.reset_timing()
+        y = d.layer_forward(0, x, k)
+        d.synchronize()
+        assert d.get_timing(1)[1] == (1 if T < 768 else 0)
+        d.set_timing(False)
+        want = orc.router_logits(L["router_w"], L["router_b"], x, E, H)
+        idx, w, logits = d.router_topk(0, x, k, want_logits=True, n_experts=E)
+        assert_bit_exact(logits, want, "router logits (canonical order)")
+        widx, ww, _, _ = orc.topk(want, k)
+        assert np.array_equal(idx, widx)
+        assert_rel_l2(w, ww, "top-k weights", 1e-6)
+        assert_rel_l2(y, orc.moe_layer(x, L, k)[0], "layer")
     finally:
         d.close()

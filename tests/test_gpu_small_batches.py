@@ -160,7 +160,8 @@ def test_small_batch_adaptive_unaligned_and_replayed(orc):
 
 
 # H: a router of one and of two loads per lane, the runtime chain (2048), padding (H < 64 NQ); T: the
-# streamed forms, the 8-token router blocks with a partial one; k: each unrolled combine and the loop
+# streamed forms, the wide router (2053 tokens; x at a 4-byte alignment: 8-token blocks with a partial
+# one); k: each unrolled combine and the loop
 @pytest.mark.parametrize("H,E,k,T", [(96, 8, 1, 5), (544, 8, 2, 40), (2048, 16, 3, 9), (2880, 8, 4, 2053), (1024, 8, 8, 33)])
 def test_block_norm_in_router_and_residual_in_combine(orc, H, E, k, T):
     """The batch's block forward gives the same bits as x + layer_forward(oracle RMSNorm(x)), also
