@@ -318,15 +318,24 @@ __global__ __launch_bounds__(kGrpThreads) void k_group(RouteArgs a, int nblk) {
   }
 }
 
-// From kRwMinTokens on: with fewer, 16-token workgroups leave most CUs idle and k_route's token per
-// workgroup is ahead (a whole layer, k_route against this, us: 320 tokens 172 / 182 at 2880 x 32
-// experts, 59.4 / 59.9 at 1024 x 8; 640 tokens 249 / 248 and 67 / 62, 87 / 86 at 2048 x 16; 1400
-// tokens 393 / 370, 85 / 67, 141 / 124). More than 32 experts would need a pass over x for each 32,
-// at which it was no faster (2048 tokens, 128 experts: 79 / 82 + 8).
-constexpr int kRwMinTokens = 768;
+// Where it is ahead of k_route: its 16-token workgroups need the tokens to fill the CUs, and k_group
+// is a launch that few entries over few experts hardly repay (a whole layer of H x I, E experts, k
+// chosen, us, k_route against this):
+//   768 tokens   3072 x 96, E 4, k 1  69.6 / 76.4;  2880 x 2880, E 8, k 1  96.9 / 101.1;  512 x 3072, E 2,
+//                k 1  68.9 / 73.3;  1024 x 512, E 16, k 2  58.1 / 54.5: behind for more shapes than not
+//   896 tokens   E k >= 8: 1024 x 512, E 8, k 4  66.6 / 59.6;  3072 x 96, E 8, k 1  75.0 / 75.4.  E k < 8:
+//                level to 4 % behind, as at 1024 tokens (3072 x 96, E 2, k 1  79.0 / 79.6, E 4 3 % behind)
+//   1100 tokens  k_route's token per workgroup, two to a CU, is in its third round: 0 to 22 % ahead
+//   2048 tokens  k_route's 8-token workgroups fill the CUs exactly once. E k < 8: 3072 x 96, E 2, k 1
+//                78.8 / 84.3, 2880 x 2880 141.6 / 147.2 (2200 tokens of 3072 x 96: 92.9 / 85.3); level from E k = 8 on
+// More than 32 experts would need a pass over x for each 32, at which it was no faster (2048 tokens,
+// 128 experts: 79 / 82 + 8).
+static bool route_wide_ahead(int T, int E, int k) {
+  return E * k < 8 ? T > 1024 && T != 2048 : T >= 896;
+}
 
 bool route_wide_fits(const RouteArgs &a) {
-  return a.T >= kRwMinTokens && a.E <= kRwMaxE && a.k <= kRwMaxK && a.H % 32 == 0 && a.H <= 128 * kGemmNs && !a.xsplit &&
+  return route_wide_ahead(a.T, a.E, a.k) && a.E <= kRwMaxE && a.k <= kRwMaxK && a.H % 32 == 0 && a.H <= 128 * kGemmNs && !a.xsplit &&
          !a.fuse_bucket && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
 }
 
@@ -347,7 +356,6 @@ hipError_t launch_route_wide(RouteArgs a, bool group, hipStream_t s) {
   switch (a.xrec ? a.rec_terms : kGemmTerms) {
     case 1: e = a.gamma ? launch_wide<1, true>(a, s) : launch_wide<1, false>(a, s); break;
     case kGemmTerms: e = a.gamma ? launch_wide<kGemmTerms, true>(a, s) : launch_wide<kGemmTerms, false>(a, s); break;
-    case kFineTerms: e = a.gamma ? launch_wide<kFineTerms, true>(a, s) : launch_wide<kFineTerms, false>(a, s); break;
   }
   if (e != hipSuccess) return e;
   if (group) {

@@ -48,12 +48,12 @@ def test_wide_router_bit_exact(orc, H, E, k, T):
         d.close()
 
 
-@pytest.mark.parametrize("T", [767, 768, 769])
-def test_switch_to_the_wide_router(orc, T):
-    """The two routers on either side of the switch give the same bits; which one ran shows in the launches:
-    32 experts' grouping does not fit k_route's LDS at this hidden size, so it needs k_bucket (kernel 1),
-    which the wide router's own grouping does without."""
-    H, E, k = 256, 32, 2
+@pytest.mark.parametrize("T,E,k", [(895, 32, 2), (896, 32, 2), (1024, 2, 1), (1025, 2, 1), (2047, 7, 1), (2048, 7, 1), (2049, 7, 1)])
+def test_switch_to_the_wide_router(orc, T, E, k):
+    """The two routers on either side of a switch give the same bits; for 32 experts, which one ran shows in
+    the launches: their grouping does not fit k_route's LDS at this hidden size, so it needs k_bucket
+    (kernel 1), which the wide router's own grouping does without."""
+    H = 256
     L = syn.make_layer(H, 96, E, seed=830, scale_lo=117, scale_hi=121, router_sigma=0.1)
     d = GpuMoeDispatcher(H, 96, 7.0)
     try:
@@ -63,7 +63,7 @@ def test_switch_to_the_wide_router(orc, T):
         d.reset_timing()
         y = d.layer_forward(0, x, k)
         d.synchronize()
-        assert d.get_timing(1)[1] == (1 if T < 768 else 0)
+        assert d.get_timing(1)[1] == (1 if E == 32 and T < 896 else 0)
         d.set_timing(False)
         want = orc.router_logits(L["router_w"], L["router_b"], x, E, H)
         idx, w, logits = d.router_topk(0, x, k, want_logits=True, n_experts=E)
