@@ -754,9 +754,11 @@ __global__ __launch_bounds__(256) void k_expert_gemv(GemvArgs a) {
 
 template <int MODE>
 static hipError_t launch_gemv_mode(const GemvArgs &a, hipStream_t s) {
-  if (!a.n_active && a.d.nq <= (uint32_t)kOneWaves) {
-    hipLaunchKernelGGL(k_expert_one<MODE>, dim3(a.d.tiles), dim3(64 * kOneWaves), 0, s, a);
-    return hipGetLastError();
+  if constexpr (MODE != GEMV_RAW) {  // (a matvec brings a list)
+    if (!a.n_active && a.d.nq <= (uint32_t)kOneWaves) {
+      hipLaunchKernelGGL(k_expert_one<MODE>, dim3(a.d.tiles), dim3(64 * kOneWaves), 0, s, a);
+      return hipGetLastError();
+    }
   }
   if (a.n_active && a.d.ns <= (uint32_t)kSmallNsMax && a.max_entries_per_expert <= 8) {
     if (a.max_entries_per_expert <= 1) return launch_small<MODE, 1>(a, s);
