@@ -632,8 +632,9 @@ hipError_t launch_gemm_stream(GemvMode mode, const GemmArgs &a, hipStream_t s, b
   return one ? launch_stream_rt<GEMV_DOWN, 2, 8, 4, 1>(a, s, n_wg) : launch_stream_rt<GEMV_DOWN, 2, 8, 4, kGemmTerms>(a, s, n_wg);
 }
 
-// The six-term form (experts averaging fewer than 4 entries). The weight stream bounds it. A register
-// rings of 4 (gate_up) and 8 (down) steps, as the three-term form's 3 and 8. Against the per-tile GEMV
+// The six-term form (experts averaging fewer than 4 entries). The weight stream bounds it. Register rings
+// of 8 steps for down, as with three terms, and 4 for gate_up (3 with three terms, and here too where the
+// step count is a run-time one). Against the per-tile GEMV
 // on bf16 hi + lo operands, whose weight decode bounds it (2880 x 2880, top-4, us per layer): 32
 // experts at 2 tokens 48.8 -> 44.5, 8 tokens 136.9 -> 85.8, 31 tokens 186.0 -> 97.4; 128 experts at
 // 16 tokens 209.8 -> 141.9, 48 tokens 462.7 -> 238.7, 127 tokens 616.9 -> 337.1. With four terms, which
